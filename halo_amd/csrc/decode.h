@@ -102,159 +102,153 @@ __device__ __forceinline__ int q3k_scale(const uint8_t* sb, uint32_t i) {
     return (int)(((sb[i % 8] >> (4 * (i / 8))) & 15u) | (((sb[8 + i % 4] >> (2 * (i / 4))) & 3u) << 4));
 }
 
-// ---- per-element decode of a GGUF row (the reference variant; byte loads) -------------------
-// Same expressions as quant.cpp; contraction is off in every caller.
-__device__ __forceinline__ float gguf_elem(uint32_t type, const uint8_t* row, uint32_t i) {
+// ---- per-element decode of a GGUF row ----------------------------------------------------------
+// Element i of a row of type T at `row` (global memory at any alignment, or a piece of the row
+// staged in LDS: EVEN says that the piece starts at a 4-byte boundary, so every 16-bit field of
+// the blocks, all of even size, is one load). Same expressions as quant.cpp.
+template <uint32_t T, bool EVEN = false>
+__device__ __forceinline__ float gguf_elem(const uint8_t* row, uint32_t i) {
 #pragma clang fp contract(off)
-    switch (type) {
-        case kF32: {
-            uint32_t u = (uint32_t)row[4 * i] | ((uint32_t)row[4 * i + 1] << 8) | ((uint32_t)row[4 * i + 2] << 16) |
-                         ((uint32_t)row[4 * i + 3] << 24);
-            return __uint_as_float(u);
+    auto ld_u16 = [](const uint8_t* p) __attribute__((always_inline)) {
+        if constexpr (EVEN) return (uint32_t)*reinterpret_cast<const uint16_t*>(p);
+        else return dev::ld_u16(p);
+    };
+    if constexpr (T == kF32 && EVEN) {
+        return *reinterpret_cast<const float*>(row + 4 * i);
+    } else if constexpr (T == kF32) {
+        const uint32_t u = (uint32_t)row[4 * i] | ((uint32_t)row[4 * i + 1] << 8) | ((uint32_t)row[4 * i + 2] << 16) |
+                     ((uint32_t)row[4 * i + 3] << 24);
+        return __uint_as_float(u);
+    } else if constexpr (T == kQ4_0) {
+        const uint8_t* blk = row + (i / 32) * 18;
+        const uint32_t e = i % 32;
+        const float d = h2f(ld_u16(blk));
+        const uint8_t b = blk[2 + (e & 15)];
+        const int q = (int)(e < 16 ? (b & 15) : (b >> 4)) - 8;
+        return (float)q * d;
+    } else if constexpr (T == kQ8_0) {
+        const uint8_t* blk = row + (i / 32) * 34;
+        const float d = h2f(ld_u16(blk));
+        return (float)(int8_t)blk[2 + i % 32] * d;
+    } else if constexpr (T == kQ4_K) {
+        const uint8_t* blk = row + (i / 256) * 144;
+        const uint32_t e = i % 256, g = e / 64, hi = (e % 64) / 32, l = e % 32;
+        const float d = h2f(ld_u16(blk)), dmin = h2f(ld_u16(blk + 2));
+        const uint8_t* s = blk + 4;
+        const uint32_t j = 2 * g + hi;
+        uint32_t sc, m;
+        if (j < 4) {
+            sc = s[j] & 63;
+            m = s[j + 4] & 63;
+        } else {
+            sc = (s[j + 4] & 15) | ((s[j - 4] >> 6) << 4);
+            m = (s[j + 4] >> 4) | ((s[j] >> 6) << 4);
         }
-        case kQ4_0: {
-            const uint8_t* blk = row + (i / 32) * 18;
-            const uint32_t e = i % 32;
-            const float d = h2f(ld_u16(blk));
-            const uint8_t b = blk[2 + (e & 15)];
-            const int q = (int)(e < 16 ? (b & 15) : (b >> 4)) - 8;
-            return (float)q * d;
+        const float d1 = d * (float)sc, m1 = dmin * (float)m;
+        const uint8_t qb = blk[16 + 32 * g + l];
+        const uint32_t q = hi ? (qb >> 4) : (qb & 15);
+        return d1 * (float)q - m1;
+    } else if constexpr (T == kQ5_K) {
+        const uint8_t* blk = row + (i / 256) * 176;
+        const uint32_t e = i % 256, g = e / 64, hi = (e % 64) / 32, l = e % 32;
+        const float d = h2f(ld_u16(blk)), dmin = h2f(ld_u16(blk + 2));
+        const uint8_t* s = blk + 4;
+        const uint32_t j = 2 * g + hi;
+        uint32_t sc, m;
+        if (j < 4) {
+            sc = s[j] & 63;
+            m = s[j + 4] & 63;
+        } else {
+            sc = (s[j + 4] & 15) | ((s[j - 4] >> 6) << 4);
+            m = (s[j + 4] >> 4) | ((s[j] >> 6) << 4);
         }
-        case kQ8_0: {
-            const uint8_t* blk = row + (i / 32) * 34;
-            const float d = h2f(ld_u16(blk));
-            return (float)(int8_t)blk[2 + i % 32] * d;
-        }
-        case kQ4_K: {
-            const uint8_t* blk = row + (i / 256) * 144;
-            const uint32_t e = i % 256, g = e / 64, hi = (e % 64) / 32, l = e % 32;
-            const float d = h2f(ld_u16(blk)), dmin = h2f(ld_u16(blk + 2));
-            const uint8_t* s = blk + 4;
-            const uint32_t j = 2 * g + hi;
-            uint32_t sc, m;
-            if (j < 4) {
-                sc = s[j] & 63;
-                m = s[j + 4] & 63;
-            } else {
-                sc = (s[j + 4] & 15) | ((s[j - 4] >> 6) << 4);
-                m = (s[j + 4] >> 4) | ((s[j] >> 6) << 4);
-            }
-            const float d1 = d * (float)sc, m1 = dmin * (float)m;
-            const uint8_t qb = blk[16 + 32 * g + l];
-            const uint32_t q = hi ? (qb >> 4) : (qb & 15);
-            return d1 * (float)q - m1;
-        }
-        case kQ5_K: {
-            const uint8_t* blk = row + (i / 256) * 176;
-            const uint32_t e = i % 256, g = e / 64, hi = (e % 64) / 32, l = e % 32;
-            const float d = h2f(ld_u16(blk)), dmin = h2f(ld_u16(blk + 2));
-            const uint8_t* s = blk + 4;
-            const uint32_t j = 2 * g + hi;
-            uint32_t sc, m;
-            if (j < 4) {
-                sc = s[j] & 63;
-                m = s[j + 4] & 63;
-            } else {
-                sc = (s[j + 4] & 15) | ((s[j - 4] >> 6) << 4);
-                m = (s[j + 4] >> 4) | ((s[j] >> 6) << 4);
-            }
-            const float d1 = d * (float)sc, m1 = dmin * (float)m;
-            const uint8_t qb = blk[48 + 32 * g + l];
-            const uint32_t q = (hi ? (qb >> 4) : (qb & 15)) + (((blk[16 + l] >> j) & 1u) ? 16u : 0u);
-            return d1 * (float)q - m1;
-        }
-        case kIQ4_XS: {
-            const uint8_t* blk = row + (i / 256) * 136;
-            const uint32_t e = i % 256, ib = e / 32, el = e % 32;
-            const float d = h2f(ld_u16(blk));
-            const uint32_t sl = (uint32_t)blk[4] | ((uint32_t)blk[5] << 8) | ((uint32_t)blk[6] << 16) | ((uint32_t)blk[7] << 24);
-            const float dl = d * (float)iq4xs_ls(ld_u16(blk + 2), sl, ib);
-            const uint8_t qb = blk[8 + 16 * ib + (el & 15)];
-            return dl * (float)iq4_value(el < 16 ? (qb & 15u) : (qb >> 4));
-        }
-        case kQ6_K: {
-            const uint8_t* blk = row + (i / 256) * 210;
-            const uint32_t e = i % 256, n = e / 128, r = e % 128, k = r / 32, l = r % 32;
-            const float d = h2f(ld_u16(blk + 208));
-            const uint8_t lb = blk[64 * n + l + 32 * (k & 1)];
-            const uint32_t lo4 = k < 2 ? (lb & 15) : (lb >> 4);
-            const uint32_t hi2 = (blk[128 + 32 * n + l] >> (2 * k)) & 3;
-            const int q = (int)(lo4 | (hi2 << 4)) - 32;
-            const float sc = (float)(int8_t)blk[192 + 8 * n + l / 16 + 2 * k];
-            return d * sc * (float)q;
-        }
-        case kF16:
-            return h2f(ld_u16(row + 2 * (uint64_t)i));
-        case kBF16:
-            return __uint_as_float(ld_u16(row + 2 * (uint64_t)i) << 16);
-        case kQ4_1: {
-            // d, m; element e < 16 the low nibble of qs[e], e + 16 the high one: fl(q) * d + m
-            const uint8_t* blk = row + (i / 32) * 20;
-            const uint32_t e = i % 32;
-            const float d = h2f(ld_u16(blk)), m = h2f(ld_u16(blk + 2));
-            const uint8_t b = blk[4 + (e & 15)];
-            const float t = (float)(e < 16 ? (b & 15) : (b >> 4)) * d;
-            return t + m;
-        }
-        case kQ5_0:
-        case kQ5_1: {
-            // the nibble as Q4_0 / Q4_1, with bit e of the 32-bit qh as its fifth bit (quant.cpp's
-            // xh_0 = bit j << 4 for e = j < 16, xh_1 = bit j + 16 << 4 for e = j + 16)
-            const bool one = type == kQ5_1;
-            const uint8_t* blk = row + (i / 32) * (one ? 24 : 22);
-            const uint32_t e = i % 32;
-            const uint8_t* qhp = blk + (one ? 4 : 2);
-            const uint32_t qh = ld_u16(qhp) | (ld_u16(qhp + 2) << 16);
-            const uint8_t b = qhp[4 + (e & 15)];
-            const uint32_t code = (e < 16 ? (b & 15u) : (b >> 4)) | (((qh >> e) & 1u) << 4);
-            const float d = h2f(ld_u16(blk));
-            if (!one) return (float)((int)code - 16) * d;
-            const float t = (float)code * d;
-            return t + h2f(ld_u16(blk + 2));
-        }
-        case kQ2_K: {
-            // element e = 128 n + 32 j + 16 h + l: code bits 2j..2j+1 of qs[32 n + 16 h + l]; scale
-            // byte 8 n + 2 j + h gives dl = d * fl(low nibble), ml = dmin * fl(high nibble)
-            const uint8_t* blk = row + (i / 256) * 84;
-            const uint32_t e = i % 256, n = e / 128, j = (e % 128) / 32, hl = (e % 32) / 16, l = e % 16;
-            const float d = h2f(ld_u16(blk + 80)), dmin = h2f(ld_u16(blk + 82));
-            const uint32_t sc = blk[8 * n + 2 * j + hl];
-            const float dl = d * (float)(sc & 15u), ml = dmin * (float)(sc >> 4);
-            const uint32_t q = (blk[16 + 32 * n + 16 * hl + l] >> (2 * j)) & 3u;
-            const float t = dl * (float)q;
-            return t - ml;
-        }
-        case kIQ4_NL: {
-            const uint8_t* blk = row + (i / 32) * 18;
-            const uint32_t e = i % 32;
-            const float d = h2f(ld_u16(blk));
-            const uint8_t qb = blk[2 + (e & 15)];
-            return d * (float)iq4_value(e < 16 ? (qb & 15u) : (qb >> 4));
-        }
-        case kQ3_K: {
-            // element e = 128 n + 32 j + l: code bits 2j..2j+1 of qs[32n + l] minus 4 unless bit
-            // 4n + j of hmask[l] is set; scale 8n + 2j + l / 16
-            const uint8_t* blk = row + (i / 256) * 110;
-            const uint32_t e = i % 256, n = e / 128, j = (e % 128) / 32, l = e % 32;
-            const float d_all = h2f(ld_u16(blk + 108));
-            const int q = (int)((blk[32 + 32 * n + l] >> (2 * j)) & 3u) - (((blk[l] >> (4 * n + j)) & 1u) ? 0 : 4);
-            const float dl = d_all * (float)(q3k_scale(blk + 96, 8 * n + 2 * j + l / 16) - 32);
-            return dl * (float)q;
-        }
-        case kIQ3_S: {
-            // sub-block b = e / 32: db = d (1 + 2 s); group k = (e % 32) / 4 takes codebook entry
-            // qs[8b + k] | (bit k of qh[b]) << 8; sign bit e % 8 of signs[4b + (e % 32) / 8]
-            const uint8_t* blk = row + (i / 256) * 110;
-            const uint32_t e = i % 256, b = e / 32, k = (e % 32) / 4;
-            const float d = h2f(ld_u16(blk));
-            const float db = d * (float)(1 + 2 * ((blk[106 + b / 2] >> (4 * (b % 2))) & 15u));
-            const uint32_t idx = blk[2 + 8 * b + k] | (((blk[66 + b] >> k) & 1u) << 8);
-            const float g = (float)((kIq3sGrid[idx] >> (8 * (e % 4))) & 0xFFu);
-            const float sgn = ((blk[74 + 4 * b + (e % 32) / 8] >> (e % 8)) & 1u) ? -1.0f : 1.0f;
-            return db * g * sgn;
-        }
-        default:
-            return 0.0f;
+        const float d1 = d * (float)sc, m1 = dmin * (float)m;
+        const uint8_t qb = blk[48 + 32 * g + l];
+        const uint32_t q = (hi ? (qb >> 4) : (qb & 15)) + (((blk[16 + l] >> j) & 1u) ? 16u : 0u);
+        return d1 * (float)q - m1;
+    } else if constexpr (T == kIQ4_XS) {
+        const uint8_t* blk = row + (i / 256) * 136;
+        const uint32_t e = i % 256, ib = e / 32, el = e % 32;
+        const float d = h2f(ld_u16(blk));
+        const uint32_t sl = (uint32_t)blk[4] | ((uint32_t)blk[5] << 8) | ((uint32_t)blk[6] << 16) | ((uint32_t)blk[7] << 24);
+        const float dl = d * (float)iq4xs_ls(ld_u16(blk + 2), sl, ib);
+        const uint8_t qb = blk[8 + 16 * ib + (el & 15)];
+        return dl * (float)iq4_value(el < 16 ? (qb & 15u) : (qb >> 4));
+    } else if constexpr (T == kQ6_K) {
+        const uint8_t* blk = row + (i / 256) * 210;
+        const uint32_t e = i % 256, n = e / 128, r = e % 128, k = r / 32, l = r % 32;
+        const float d = h2f(ld_u16(blk + 208));
+        const uint8_t lb = blk[64 * n + l + 32 * (k & 1)];
+        const uint32_t lo4 = k < 2 ? (lb & 15) : (lb >> 4);
+        const uint32_t hi2 = (blk[128 + 32 * n + l] >> (2 * k)) & 3;
+        const int q = (int)(lo4 | (hi2 << 4)) - 32;
+        const float sc = (float)(int8_t)blk[192 + 8 * n + l / 16 + 2 * k];
+        return d * sc * (float)q;
+    } else if constexpr (T == kF16) {
+        return h2f(ld_u16(row + 2 * (uint64_t)i));
+    } else if constexpr (T == kBF16) {
+        return __uint_as_float(ld_u16(row + 2 * (uint64_t)i) << 16);
+    } else if constexpr (T == kQ4_1) {
+        // d, m; element e < 16 the low nibble of qs[e], e + 16 the high one: fl(q) * d + m
+        const uint8_t* blk = row + (i / 32) * 20;
+        const uint32_t e = i % 32;
+        const float d = h2f(ld_u16(blk)), m = h2f(ld_u16(blk + 2));
+        const uint8_t b = blk[4 + (e & 15)];
+        const float t = (float)(e < 16 ? (b & 15) : (b >> 4)) * d;
+        return t + m;
+    } else if constexpr (T == kQ5_0 || T == kQ5_1) {
+        // the nibble as Q4_0 / Q4_1, with bit e of the 32-bit qh as its fifth bit (quant.cpp's
+        // xh_0 = bit j << 4 for e = j < 16, xh_1 = bit j + 16 << 4 for e = j + 16)
+        constexpr bool one = T == kQ5_1;
+        const uint8_t* blk = row + (i / 32) * (one ? 24 : 22);
+        const uint32_t e = i % 32;
+        const uint8_t* qhp = blk + (one ? 4 : 2);
+        const uint32_t qh = ld_u16(qhp) | (ld_u16(qhp + 2) << 16);
+        const uint8_t b = qhp[4 + (e & 15)];
+        const uint32_t code = (e < 16 ? (b & 15u) : (b >> 4)) | (((qh >> e) & 1u) << 4);
+        const float d = h2f(ld_u16(blk));
+        if (!one) return (float)((int)code - 16) * d;
+        const float t = (float)code * d;
+        return t + h2f(ld_u16(blk + 2));
+    } else if constexpr (T == kQ2_K) {
+        // element e = 128 n + 32 j + 16 h + l: code bits 2j..2j+1 of qs[32 n + 16 h + l]; scale
+        // byte 8 n + 2 j + h gives dl = d * fl(low nibble), ml = dmin * fl(high nibble)
+        const uint8_t* blk = row + (i / 256) * 84;
+        const uint32_t e = i % 256, n = e / 128, j = (e % 128) / 32, hl = (e % 32) / 16, l = e % 16;
+        const float d = h2f(ld_u16(blk + 80)), dmin = h2f(ld_u16(blk + 82));
+        const uint32_t sc = blk[8 * n + 2 * j + hl];
+        const float dl = d * (float)(sc & 15u), ml = dmin * (float)(sc >> 4);
+        const uint32_t q = (blk[16 + 32 * n + 16 * hl + l] >> (2 * j)) & 3u;
+        const float t = dl * (float)q;
+        return t - ml;
+    } else if constexpr (T == kIQ4_NL) {
+        const uint8_t* blk = row + (i / 32) * 18;
+        const uint32_t e = i % 32;
+        const float d = h2f(ld_u16(blk));
+        const uint8_t qb = blk[2 + (e & 15)];
+        return d * (float)iq4_value(e < 16 ? (qb & 15u) : (qb >> 4));
+    } else if constexpr (T == kQ3_K) {
+        // element e = 128 n + 32 j + l: code bits 2j..2j+1 of qs[32n + l] minus 4 unless bit
+        // 4n + j of hmask[l] is set; scale 8n + 2j + l / 16
+        const uint8_t* blk = row + (i / 256) * 110;
+        const uint32_t e = i % 256, n = e / 128, j = (e % 128) / 32, l = e % 32;
+        const float d_all = h2f(ld_u16(blk + 108));
+        const int q = (int)((blk[32 + 32 * n + l] >> (2 * j)) & 3u) - (((blk[l] >> (4 * n + j)) & 1u) ? 0 : 4);
+        const float dl = d_all * (float)(q3k_scale(blk + 96, 8 * n + 2 * j + l / 16) - 32);
+        return dl * (float)q;
+    } else if constexpr (T == kIQ3_S) {
+        // sub-block b = e / 32: db = d (1 + 2 s); group k = (e % 32) / 4 takes codebook entry
+        // qs[8b + k] | (bit k of qh[b]) << 8; sign bit e % 8 of signs[4b + (e % 32) / 8]
+        const uint8_t* blk = row + (i / 256) * 110;
+        const uint32_t e = i % 256, b = e / 32, k = (e % 32) / 4;
+        const float d = h2f(ld_u16(blk));
+        const float db = d * (float)(1 + 2 * ((blk[106 + b / 2] >> (4 * (b % 2))) & 15u));
+        const uint32_t idx = blk[2 + 8 * b + k] | (((blk[66 + b] >> k) & 1u) << 8);
+        const float g = (float)((kIq3sGrid[idx] >> (8 * (e % 4))) & 0xFFu);
+        const float sgn = ((blk[74 + 4 * b + (e % 32) / 8] >> (e % 8)) & 1u) ? -1.0f : 1.0f;
+        return db * g * sgn;
+    } else {
+        static_assert(T == kF32, "a type of the GGUF layout");
     }
 }
 

@@ -19,44 +19,6 @@ namespace {
 using namespace dev;
 
 // ==========================================================================================
-// Reference-order GEMV over GGUF rows (bitwise equal to cpu::matmul)
-// ==========================================================================================
-
-// Block of 256 threads = 32 groups of 8 lanes; group -> one W row, every x vector.
-__global__ __launch_bounds__(256) void k_gemv_gguf_ref(uint32_t type, const uint8_t* __restrict__ w, uint64_t w_stride,
-                                                       const float* __restrict__ x, uint64_t x_stride,
-                                                       float* __restrict__ y, uint64_t y_stride, uint32_t rows,
-                                                       uint32_t cols, uint32_t n_vec) {
-#pragma clang fp contract(off)
-    const uint32_t j = threadIdx.x & 7u;
-    const uint32_t n = blockIdx.x * 32u + (threadIdx.x >> 3);
-    const bool live = n < rows;
-    const uint8_t* row = w + (uint64_t)(live ? n : 0) * w_stride;
-    const uint32_t full = cols - cols % 8u;
-    for (uint32_t t = 0; t < n_vec; ++t) {
-        const float* xt = x + (uint64_t)t * x_stride;
-        float p = 0.0f;
-        if (live)
-            for (uint32_t i = j; i < full; i += 8) {
-                const float prod = xt[i] * gguf_elem(type, row, i);
-                p = p + prod;
-            }
-        // ((p0+p4)+(p1+p5)) + ((p2+p6)+(p3+p7)), then + tail, exactly as the CPU dot.
-        const float q = p + __shfl_down(p, 4, 8);   // lanes 0..3: p_j + p_{j+4}
-        const float r = q + __shfl_down(q, 1, 8);   // lane 0: left, lane 2: right
-        const float s = r + __shfl_down(r, 2, 8);   // lane 0: left + right
-        if (j == 0 && live) {
-            float tail = 0.0f;
-            for (uint32_t i = full; i < cols; ++i) {
-                const float prod = xt[i] * gguf_elem(type, row, i);
-                tail = tail + prod;
-            }
-            y[(uint64_t)t * y_stride + n] = s + tail;
-        }
-    }
-}
-
-// ==========================================================================================
 // SLAB GEMV: one row per lane; a one-wave workgroup owns a (slab, K chunk) unit
 // ==========================================================================================
 //

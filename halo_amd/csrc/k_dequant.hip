@@ -96,7 +96,8 @@ __device__ __forceinline__ bool table_row(const int32_t* ids, uint32_t table_row
     return true;
 }
 
-__global__ void k_dequant_gguf(uint32_t type, const uint8_t* __restrict__ w, uint64_t w_stride, uint32_t cols,
+template <uint32_t T>
+__global__ void k_dequant_gguf(const uint8_t* __restrict__ w, uint64_t w_stride, uint32_t cols,
                                uint32_t first_row, uint32_t n_rows, float* __restrict__ out, uint64_t out_stride,
                                const int32_t* __restrict__ ids, uint32_t table_rows, uint32_t* status) {
     const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -105,7 +106,7 @@ __global__ void k_dequant_gguf(uint32_t type, const uint8_t* __restrict__ w, uin
     const uint32_t i = (uint32_t)(idx % cols);
     uint64_t row;
     if (!table_row(ids, table_rows, first_row, r, i == 0, status, row)) return;
-    out[r * out_stride + i] = gguf_elem(type, w + row * w_stride, i);
+    out[r * out_stride + i] = gguf_elem<T>(w + row * w_stride, i);
 }
 
 // Exact fp32 weights of slot s of the row at lane r of `slab` (the reference's expressions).
@@ -277,8 +278,28 @@ int launch_dequant_gguf(uint32_t type, const uint8_t* w, uint64_t w_stride, uint
                         uint32_t n_rows, float* out, uint64_t out_stride, hipStream_t st, const int32_t* ids,
                         uint32_t table_rows, uint32_t* status) {
     const uint64_t n = (uint64_t)n_rows * cols;
-    hipLaunchKernelGGL(k_dequant_gguf, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, st, type, w, w_stride, cols,
-                       first_row, n_rows, out, out_stride, ids, table_rows, status);
+    const dim3 grid((uint32_t)((n + 255) / 256)), block(256);
+#define HALO_MI_DQ(T) case T: hipLaunchKernelGGL(k_dequant_gguf<T>, grid, block, 0, st, w, w_stride, cols, first_row, n_rows, out, out_stride, ids, table_rows, status); break
+    switch (type) {
+        HALO_MI_DQ(kF32);
+        HALO_MI_DQ(kF16);
+        HALO_MI_DQ(kBF16);
+        HALO_MI_DQ(kQ4_0);
+        HALO_MI_DQ(kQ4_1);
+        HALO_MI_DQ(kQ5_0);
+        HALO_MI_DQ(kQ5_1);
+        HALO_MI_DQ(kQ8_0);
+        HALO_MI_DQ(kQ2_K);
+        HALO_MI_DQ(kQ3_K);
+        HALO_MI_DQ(kQ4_K);
+        HALO_MI_DQ(kQ5_K);
+        HALO_MI_DQ(kQ6_K);
+        HALO_MI_DQ(kIQ4_NL);
+        HALO_MI_DQ(kIQ3_S);
+        HALO_MI_DQ(kIQ4_XS);
+        default: return set_error(HALO_MI_E_UNSUPPORTED, "dequant: type %u has no decoder", type);
+    }
+#undef HALO_MI_DQ
     return hip_status(hipGetLastError(), "dequant_gguf launch");
 }
 

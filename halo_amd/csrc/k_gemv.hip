@@ -1,7 +1,4 @@
 // gfx950 GEMV kernels of the halo_mi355x library (M = 1..8):
-//   k_gemv_gguf_ref  GGUF layout, 8 lanes per output in cpu::detail::dot's order
-//                    (backends/cpu/kernel_common.h:16-27 of the reference): bit-identical to the
-//                    CPU backend.
 //   k_gemv_slab      SLAB layout, VALU: one row per lane, a wave streams 64 rows slot by slot.
 //   k_gemv_mx        SLAB layout, the same stream with the multiply-adds on
 //                    v_mfma_f32_4x4x4_16b_bf16 (the default).
@@ -433,14 +430,3 @@ extern "C" int halo_mi_gemv_noalloc(const halo_mi_gemv_params* p, void* stream) 
     a.valu = v == HALO_MI_GEMV_SLAB_VALU;
     return launch_gemv_slab_in<false>(p->type, a, &ws, kNaSlots, kNaCounters, kNaNormFloats, static_cast<hipStream_t>(stream));
 }
-
-namespace halo_mi {
-
-int launch_gemv_gguf_ref(uint32_t type, const uint8_t* w, uint64_t w_stride, const float* x, uint64_t x_stride, float* y,
-                         uint64_t y_stride, uint32_t rows, uint32_t cols, uint32_t n_vec, hipStream_t st) {
-    hipLaunchKernelGGL(k_gemv_gguf_ref, dim3((rows + 31) / 32), dim3(256), 0, st, type, w, w_stride, x, x_stride, y,
-                       y_stride, rows, cols, n_vec);
-    return hip_status(hipGetLastError(), "gemv_gguf_ref launch");
-}
-
-}  // namespace halo_mi

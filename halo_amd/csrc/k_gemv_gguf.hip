@@ -1,0 +1,293 @@
+// gfx950 reference-order GEMV of the halo_mi355x library (HALO_MI_GEMV_GGUF_REF): GGUF rows of any
+// of the 16 types at any alignment, 8 sums per output in cpu::detail::dot's order
+// (backends/cpu/kernel_common.h:16-27 of the reference), so y is bit-identical to the CPU backend.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cstdint>
+
+#include "device.h"
+#include "launch.h"
+
+namespace halo_mi {
+namespace {
+
+using namespace dev;
+
+// What bounds it: the CPU's order leaves 8 independent sums per output, each a chain of cols / 8
+// products added one at a time, with the product rounded before its addition (no fused
+// multiply-add). So the kernel is bound by vector instructions (decode, multiply, add), not by HBM.
+//
+// Lane l of a wave holds sum j = l % 8 of the rows l / 8 + 8 i, i < R, for NV vectors. Per chunk of
+// CH elements of K:
+//   - the wave brings its rows' bytes into its own piece of LDS with 16-byte loads at whatever
+//     alignment the rows have (the next chunk's loads are in flight while this one is computed);
+//   - the workgroup stages x in LDS by sum: element 8 s + j of a vector at [j][s], so the four
+//     products of a 32-element slot that lane j takes (elements j, j + 8, j + 16, j + 24) need one
+//     16-byte read; two buffers, one barrier per chunk;
+//   - every weight is decoded once per launch and vector group and used for NV vectors.
+// With 8 or 16 vectors a lane takes two rows (when that still fills the chip), so each 16-byte read
+// of x feeds 16 instructions: with one row the LDS path (8 cycles per read and CU) and the four
+// SIMDs' 8 multiply-adds would be equally busy.
+//
+// Measured on MI355X against one thread per sum with byte loads and every weight decoded once per
+// vector: IQ4_NL 5120 x 17408 at 1 vector 646 -> 62 us, Q3_K 17408 x 5120 at 64 vectors 14470 ->
+// 439 us (13 T multiply-adds/s; the two rounded operations alone take about 290 us).
+template <uint32_t T, int NV>
+constexpr uint32_t chunk_elems() {
+    // at most 640 bytes of a row and 16 x loads per thread and chunk
+    uint32_t ch = NV == 1 ? 1024u : NV == 2 ? 512u : 256u;
+    while (ch / block_elems(T) * block_bytes(T) > 640 && ch > 128 && ch / 2 % block_elems(T) == 0) ch /= 2;
+    return ch;
+}
+
+// Threads per workgroup: single waves for few vectors (8 rows each, so 5120 rows are 640 workgroups
+// over 256 CUs; four-wave workgroups would leave 96 CUs idle), four for many (they share x).
+template <int NV>
+constexpr uint32_t ref_threads() {
+    return NV <= 4 ? 64u : 256u;
+}
+
+// The weights of elements j, j + 8, j + 16, j + 24 of slot `s` (32 elements) of the row piece `row`.
+template <uint32_t T>
+__device__ __forceinline__ void slot4(const uint8_t* row, uint32_t s, uint32_t j, float w[4]) {
+#pragma clang fp contract(off)
+    if constexpr (T == kIQ4_NL || T == kIQ4_XS) {
+        // bytes j and j + 8 of the slot's 16 code bytes; four table lookups at once
+        constexpr bool xs = T == kIQ4_XS;
+        const uint8_t* blk = xs ? row + s / 8 * 136 : row + s * 18;
+        const uint8_t* qs = xs ? blk + 8 + 16 * (s % 8) : blk + 2;
+        const float d0 = h2f(*reinterpret_cast<const uint16_t*>(blk));
+        float d = d0;
+        if constexpr (xs)
+            d = d0 * (float)iq4xs_ls(*reinterpret_cast<const uint16_t*>(blk + 2), *reinterpret_cast<const uint32_t*>(blk + 4), s % 8);
+        const uint32_t q = (uint32_t)qs[j] | ((uint32_t)qs[j + 8] << 8);
+        const uint32_t v = iq4_lookup4((q & 0x0F0Fu) | ((q & 0xF0F0u) << 12));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) w[k] = d * (ubyte(v, k) - 128.0f);
+    } else {
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) w[k] = gguf_elem<T, true>(row, 32 * s + j + 8 * k);
+    }
+}
+
+// 16 bytes at p of which `avail` may be read (the others come back as zero).
+__device__ __forceinline__ uint4 load_piece(const uint8_t* p, uint64_t avail) {
+    uint4 v{0, 0, 0, 0};
+    if (avail >= 16) {
+        __builtin_memcpy(&v, p, 16);
+    } else {
+        uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (uint32_t b = 0; b < 15; ++b)
+            if (b < avail) w[b / 4] |= (uint32_t)p[b] << (8 * (b % 4));
+        v = uint4{w[0], w[1], w[2], w[3]};
+    }
+    return v;
+}
+
+template <uint32_t T, int NV, int R>
+__global__ __launch_bounds__(ref_threads<NV>()) void k_gemv_gguf_ref(const uint8_t* __restrict__ w, uint64_t w_stride,
+                                                                     const float* __restrict__ x, uint64_t x_stride,
+                                                                     float* __restrict__ y, uint64_t y_stride, uint32_t rows,
+                                                                     uint32_t cols, uint32_t n_vec) {
+#pragma clang fp contract(off)
+    constexpr uint32_t BE = block_elems(T), BB = block_bytes(T), TH = ref_threads<NV>(), WAVES = TH / 64;
+    constexpr uint32_t CH = chunk_elems<T, NV>(), CHB = CH / BE * BB;
+    constexpr uint32_t PIECES = (CHB + 15) / 16, WR = 8 * R, NLD = (WR * PIECES + 63) / 64;
+    constexpr uint32_t RS = PIECES * 16 + 16;  // LDS bytes of a row's piece: the rows start on different banks
+    constexpr uint32_t XS = CH / 8 + 4;        // LDS floats of one sum's x: the 8 sums start on different banks
+    constexpr uint32_t XLD = NV * CH / TH;     // x loads per thread and chunk
+    static_assert(NV * CH % TH == 0 && CH % 32 == 0 && CH % BE == 0 && XS % 4 == 0);
+    __shared__ __align__(16) uint8_t wl[WAVES][WR * RS];
+    __shared__ __align__(16) float xl[2][NV * 8 * XS];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, j = lane & 7u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t row0 = (blockIdx.x * WAVES + wave) * WR, t0 = blockIdx.y * NV;
+    const uint32_t full = cols - cols % 8u, nch = full / CH + (full % CH != 0);
+    const uint64_t row_len = (uint64_t)(cols / BE) * BB;
+
+    uint4 wreg[NLD];
+    float xreg[XLD];
+    auto load = [&](uint32_t c) __attribute__((always_inline)) {
+        const uint64_t b0 = (uint64_t)c * CHB, left = row_len - b0;
+        const uint32_t here = (uint32_t)min((uint64_t)CHB, left);  // this chunk's bytes of a row
+#pragma unroll
+        for (uint32_t i = 0; i < NLD; ++i) {
+            const uint32_t e = lane + 64 * i, r = e / PIECES, o = e % PIECES * 16;
+            wreg[i] = uint4{0, 0, 0, 0};
+            if (r < WR && o < here)  // rows past the end read the last row; their sums are not stored
+                wreg[i] = load_piece(w + (uint64_t)min(row0 + r, rows - 1) * w_stride + b0 + o, left - o);
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < XLD; ++i) {
+            const uint32_t e = tid + TH * i, v = e / CH, k = c * CH + e % CH;
+            xreg[i] = k < full ? x[(uint64_t)min(t0 + v, n_vec - 1) * x_stride + k] : 0.0f;
+        }
+    };
+    auto store = [&](uint32_t c) __attribute__((always_inline)) {
+#pragma unroll
+        for (uint32_t i = 0; i < NLD; ++i) {
+            const uint32_t e = lane + 64 * i, r = e / PIECES, o = e % PIECES * 16;
+            if (r < WR) *reinterpret_cast<uint4*>(&wl[wave][r * RS + o]) = wreg[i];
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < XLD; ++i) {
+            const uint32_t e = tid + TH * i, v = e / CH, k = e % CH;
+            xl[c & 1u][(v * 8 + k % 8) * XS + k / 8] = xreg[i];
+        }
+    };
+
+    float p[R][NV];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int v = 0; v < NV; ++v) p[r][v] = 0.0f;
+    if (nch > 0) {
+        load(0);
+        store(0);
+    }
+    __syncthreads();
+    for (uint32_t c = 0; c < nch; ++c) {
+        if (c + 1 < nch) load(c + 1);
+        const uint32_t steps = min(CH, full - c * CH) / 8;  // additions of each sum in this chunk
+        const uint8_t* rp = &wl[wave][lane / 8 * RS];
+        const float* xp = &xl[c & 1u][j * XS];
+        auto slot = [&](const uint8_t* piece, uint32_t sl, uint32_t s) __attribute__((always_inline)) {
+            float q[R][4];
+#pragma unroll
+            for (int r = 0; r < R; ++r) slot4<T>(piece + r * 8 * RS, sl, j, q[r]);
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                const float4 xv = *reinterpret_cast<const float4*>(xp + v * 8 * XS + 4 * s);
+                const float xe[4] = {xv.x, xv.y, xv.z, xv.w};
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        const float prod = xe[k] * q[r][k];
+                        p[r][v] = p[r][v] + prod;
+                    }
+            }
+        };
+        if constexpr (BE == 256) {
+            for (uint32_t b = 0; b < steps / 32; ++b)
+#pragma unroll
+                for (uint32_t sl = 0; sl < 8; ++sl) slot(rp + b * BB, sl, b * 8 + sl);
+        } else {
+#pragma unroll 4
+            for (uint32_t s = 0; s < steps / 4; ++s) slot(rp + s * (32 / BE * BB), 0, s);
+            if constexpr (BE == 1) {  // a last slot of fewer than four additions
+                for (uint32_t k = steps & ~3u; k < steps; ++k)
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        const float q = gguf_elem<T, true>(rp + r * 8 * RS, 8 * k + j);
+#pragma unroll
+                        for (int v = 0; v < NV; ++v) {
+                            const float prod = xp[v * 8 * XS + k] * q;
+                            p[r][v] = p[r][v] + prod;
+                        }
+                    }
+            }
+        }
+        if (c + 1 < nch) store(c + 1);
+        __syncthreads();
+    }
+    // ((p0+p4)+(p1+p5)) + ((p2+p6)+(p3+p7)), then + tail, exactly as the CPU dot
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const float a = p[r][v] + __shfl_down(p[r][v], 4, 8);  // lanes 0..3: p_j + p_{j+4}
+            const float b = a + __shfl_down(a, 1, 8);              // lane 0: left, lane 2: right
+            const float s = b + __shfl_down(b, 2, 8);              // lane 0: left + right
+            const uint32_t n = row0 + 8 * r + lane / 8;
+            if (j == 0 && n < rows && t0 + v < n_vec) {
+                const float* xt = x + (uint64_t)(t0 + v) * x_stride;
+                float tail = 0.0f;
+                if constexpr (BE == 1)
+                    for (uint32_t i = full; i < cols; ++i) {
+                        const float prod = xt[i] * gguf_elem<T>(w + (uint64_t)n * w_stride, i);
+                        tail = tail + prod;
+                    }
+                y[(uint64_t)(t0 + v) * y_stride + n] = s + tail;
+            }
+        }
+}
+
+struct RefArgs {
+    const uint8_t* w;
+    uint64_t w_stride;
+    const float* x;
+    uint64_t x_stride;
+    float* y;
+    uint64_t y_stride;
+    uint32_t rows, cols;
+};
+
+// `n` vectors from t0 on, NV per workgroup (the last group may be short)
+template <uint32_t T, int NV, int R>
+void launch_ref_nv(const RefArgs& a, uint32_t t0, uint32_t n, hipStream_t st) {
+    constexpr uint32_t per = ref_threads<NV>() / 64 * 8 * R;  // rows per workgroup
+    constexpr uint32_t kMaxGroups = 32768;                    // grid.y stays within the launch limits
+    for (uint32_t k = 0; k < n; k += kMaxGroups * NV) {
+        const uint32_t m = std::min(n - k, kMaxGroups * NV);
+        hipLaunchKernelGGL((k_gemv_gguf_ref<T, NV, R>), dim3((a.rows - 1) / per + 1, (m + NV - 1) / NV), dim3(ref_threads<NV>()),
+                           0, st, a.w, a.w_stride, a.x + (uint64_t)(t0 + k) * a.x_stride, a.x_stride,
+                           a.y + (uint64_t)(t0 + k) * a.y_stride, a.y_stride, a.rows, a.cols, m);
+    }
+}
+
+template <uint32_t T>
+void launch_ref(const RefArgs& a, uint32_t n_vec, hipStream_t st) {
+    // groups of 16 vectors, then the smallest form that takes the rest in one launch
+    const uint32_t many = n_vec / 16 * 16, rest = n_vec - many;
+    // two rows per lane once that leaves about one wave per SIMD (1024 SIMDs x 16 rows)
+    const auto two = [&](uint32_t groups) { return (uint64_t)a.rows * groups >= 16 * 1024; };
+    if (many) {
+        if (two(many / 16)) launch_ref_nv<T, 16, 2>(a, 0, many, st);
+        else launch_ref_nv<T, 16, 1>(a, 0, many, st);
+    }
+    if (rest > 8) {
+        if (two(1)) launch_ref_nv<T, 16, 2>(a, many, rest, st);
+        else launch_ref_nv<T, 16, 1>(a, many, rest, st);
+    } else if (rest > 4) {
+        if (two(1)) launch_ref_nv<T, 8, 2>(a, many, rest, st);
+        else launch_ref_nv<T, 8, 1>(a, many, rest, st);
+    } else if (rest > 2) {
+        launch_ref_nv<T, 4, 1>(a, many, rest, st);
+    } else if (rest == 2) {
+        launch_ref_nv<T, 2, 1>(a, many, rest, st);
+    } else if (rest == 1) {
+        launch_ref_nv<T, 1, 1>(a, many, rest, st);
+    }
+}
+
+}  // namespace
+
+int launch_gemv_gguf_ref(uint32_t type, const uint8_t* w, uint64_t w_stride, const float* x, uint64_t x_stride, float* y,
+                         uint64_t y_stride, uint32_t rows, uint32_t cols, uint32_t n_vec, hipStream_t st) {
+    const RefArgs a{w, w_stride, x, x_stride, y, y_stride, rows, cols};
+    switch (type) {
+        case kF32: launch_ref<kF32>(a, n_vec, st); break;
+        case kF16: launch_ref<kF16>(a, n_vec, st); break;
+        case kBF16: launch_ref<kBF16>(a, n_vec, st); break;
+        case kQ4_0: launch_ref<kQ4_0>(a, n_vec, st); break;
+        case kQ4_1: launch_ref<kQ4_1>(a, n_vec, st); break;
+        case kQ5_0: launch_ref<kQ5_0>(a, n_vec, st); break;
+        case kQ5_1: launch_ref<kQ5_1>(a, n_vec, st); break;
+        case kQ8_0: launch_ref<kQ8_0>(a, n_vec, st); break;
+        case kQ2_K: launch_ref<kQ2_K>(a, n_vec, st); break;
+        case kQ3_K: launch_ref<kQ3_K>(a, n_vec, st); break;
+        case kQ4_K: launch_ref<kQ4_K>(a, n_vec, st); break;
+        case kQ5_K: launch_ref<kQ5_K>(a, n_vec, st); break;
+        case kQ6_K: launch_ref<kQ6_K>(a, n_vec, st); break;
+        case kIQ4_NL: launch_ref<kIQ4_NL>(a, n_vec, st); break;
+        case kIQ3_S: launch_ref<kIQ3_S>(a, n_vec, st); break;
+        case kIQ4_XS: launch_ref<kIQ4_XS>(a, n_vec, st); break;
+        default: return set_error(HALO_MI_E_UNSUPPORTED, "gemv_gguf_ref: type %u has no decoder", type);
+    }
+    return hip_status(hipGetLastError(), "gemv_gguf_ref launch");
+}
+
+}  // namespace halo_mi

@@ -1,0 +1,66 @@
+"""The reference-order GEMV at the edges of its forms: the vector groups (1, 2, 4, 8, 16 vectors and what is
+left over), one or two rows per lane, the K chunks and their remainders, and rows at any byte alignment and
+stride. Every result is bitwise cpu::matmul (the oracle)."""
+import numpy as np
+import pytest
+
+from helpers import (BLOCK, F16, F32, GGUF_TYPES, IQ4_NL, NAMES, PLAIN_TYPES, Q3_K, Q6_K, Q8_0, isclose_bits, make_weights)
+from test_gpu_parity import run_gemv, say, to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+def check(hl, oracle, dev, t, rows, cols, n_vec, pad=0, off=0, xp=0, yp=0, scale=1.0):
+    say("gguf rows", NAMES[t], rows, cols, n_vec, pad, off)
+    buf, stride = make_weights(t, rows, cols, seed=7 + t + rows + n_vec, stride_pad=pad, offset=off)
+    x = (np.random.default_rng(n_vec + cols).uniform(-1, 1, (n_vec, cols)) * scale).astype(np.float32)
+    x[0, 0] = -0.0
+    ref = oracle.matmul(t, buf[off:], rows, cols, x, w_stride=stride)
+    wd = to_dev(buf, dev)
+    y = run_gemv(hl, dev, t, wd.data_ptr() + off, hl.Layout.GGUF, x, rows, cols, hl.Variant.DEFAULT, xp, yp, stride)
+    assert isclose_bits(y, ref)
+
+
+@pytest.mark.parametrize("t", GGUF_TYPES)
+@pytest.mark.parametrize("n_vec", [1, 2, 3, 5, 9, 17, 40])
+def test_vector_groups(hl, oracle, dev, t, n_vec):
+    # 1280 columns: a whole 1024-element chunk and a part of one; 9 rows: a wave's 8 and one more
+    pad, off = (4, 4) if t == F32 else (3, 1)  # (F32 rows are 4-byte aligned)
+    check(hl, oracle, dev, t, 9, 1280, n_vec, pad=pad, off=off, xp=1, yp=5)
+
+
+@pytest.mark.parametrize("t", [Q3_K, Q6_K, IQ4_NL, Q8_0, F16, F32])
+@pytest.mark.parametrize("n_vec", [7, 16])
+def test_two_rows_per_lane(hl, oracle, dev, t, n_vec):
+    # 16385 rows: the two-row forms, one row past a whole workgroup of 64
+    check(hl, oracle, dev, t, 16385, BLOCK[t][0] if BLOCK[t][0] > 32 else 32, n_vec)
+
+
+@pytest.mark.parametrize("t", PLAIN_TYPES)
+@pytest.mark.parametrize("cols", [1, 7, 8, 9, 31, 33, 135, 257, 1031])
+@pytest.mark.parametrize("n_vec", [1, 6])
+def test_ragged_columns(hl, oracle, dev, t, cols, n_vec):
+    check(hl, oracle, dev, t, 17, cols, n_vec, off=4 if t == F32 else 2)
+
+
+@pytest.mark.parametrize("t", [IQ4_NL, Q8_0])
+@pytest.mark.parametrize("cols", [32, 96, 1056, 2080])
+def test_short_blocks(hl, oracle, dev, t, cols):
+    check(hl, oracle, dev, t, 33, cols, 1, pad=1)
+    check(hl, oracle, dev, t, 33, cols, 4, scale=2.0 ** 60)
+
+
+@pytest.mark.parametrize("t", [IQ4_NL, F16])
+def test_infinities_and_nan(hl, oracle, dev, t):
+    """A non-finite x reaches only its own vector's outputs, as on the CPU."""
+    rows, cols = 24, 512
+    buf, stride = make_weights(t, rows, cols, seed=5)
+    x = np.random.default_rng(3).uniform(-1, 1, (3, cols)).astype(np.float32)
+    x[1, 37] = np.inf
+    x[2, 500] = np.nan
+    ref = oracle.matmul(t, buf, rows, cols, x)
+    wd = to_dev(buf, dev)
+    y = run_gemv(hl, dev, t, wd.data_ptr(), hl.Layout.GGUF, x, rows, cols, hl.Variant.DEFAULT, 0, 0, stride)
+    assert isclose_bits(y[0], ref[0])
+    assert np.array_equal(np.isnan(y), np.isnan(ref))
+    assert np.array_equal(y[~np.isnan(ref)], ref[~np.isnan(ref)])
