@@ -96,126 +96,108 @@ __device__ __forceinline__ bool table_row(const int32_t* ids, uint32_t table_row
     return true;
 }
 
-template <uint32_t T>
-__global__ void k_dequant_gguf(const uint8_t* __restrict__ w, uint64_t w_stride, uint32_t cols,
-                               uint32_t first_row, uint32_t n_rows, float* __restrict__ out, uint64_t out_stride,
-                               const int32_t* __restrict__ ids, uint32_t table_rows, uint32_t* status) {
-    const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (uint64_t)n_rows * cols) return;
-    const uint64_t r = idx / cols;
-    const uint32_t i = (uint32_t)(idx % cols);
-    uint64_t row;
-    if (!table_row(ids, table_rows, first_row, r, i == 0, status, row)) return;
-    out[r * out_stride + i] = gguf_elem<T>(w + row * w_stride, i);
-}
+// Dequantize / GET_ROWS: a block of kDqThreads threads takes kDqElems consecutive elements of one
+// output row (blocks of a row follow each other, so the row's index is one scalar division), four
+// consecutive elements per thread: a wave stores 1 KB at once. Bound by launch and load latency at
+// a prefill chunk's sizes: 512 rows of 5120 from a Q6_K SLAB table 7.9 -> 5.7 us (one thread per
+// 32-element slot stored 4 bytes at a 128-byte pitch), from a GGUF table 8.7 -> 6.5 us (one thread
+// per element with 64-bit divisions); Q4_K 7.2 -> 4.7 and 8.8 -> 6.3.
+constexpr uint32_t kDqThreads = 256, kDqElems = 4 * kDqThreads;
 
-// Exact fp32 weights of slot s of the row at lane r of `slab` (the reference's expressions).
-template <uint32_t T>
-__device__ __forceinline__ void slab_slot_weights(const uint8_t* __restrict__ slab, const SlabGeom& g, uint32_t r,
-                                                  uint32_t s, float w[32]) {
-#pragma clang fp contract(off)
-    if constexpr (T == kQ4_0) {
-        const uint4 q = *reinterpret_cast<const uint4*>(slab + g.q_off + ((uint64_t)s * 64 + r) * 16);
-        const float d = h2f(*reinterpret_cast<const uint16_t*>(slab + g.aux_off + ((uint64_t)s * 64 + r) * 2));
-        const uint32_t Q[4] = {q.x, q.y, q.z, q.w};
+// Stores w[0..3] at o[i..i+3], of which the first `left` exist; 16-byte stores where the row is aligned.
+__device__ __forceinline__ void store4(float* o, uint32_t i, uint32_t left, const float w[4]) {
+    if (left >= 4 && (reinterpret_cast<uintptr_t>(o + i) & 15u) == 0) {
+        *reinterpret_cast<float4*>(o + i) = float4{w[0], w[1], w[2], w[3]};
+    } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const uint32_t b = (Q[i] >> (8 * k)) & 0xFFu;
-                w[4 * i + k] = (float)((int)(b & 15u) - 8) * d;
-                w[16 + 4 * i + k] = (float)((int)(b >> 4) - 8) * d;
-            }
-    } else if constexpr (T == kQ8_0) {
-        const float d = h2f(*reinterpret_cast<const uint16_t*>(slab + g.aux_off + ((uint64_t)s * 64 + r) * 2));
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const uint4 q = *reinterpret_cast<const uint4*>(slab + g.q_off + (((uint64_t)s * 2 + h) * 64 + r) * 16);
-            const uint32_t Q[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int k = 0; k < 4; ++k) w[16 * h + 4 * i + k] = sbyte(Q[i], k) * d;
-        }
-    } else if constexpr (T == kQ4_K) {
-        const uint4 q = *reinterpret_cast<const uint4*>(slab + g.q_off + ((uint64_t)s * 64 + r) * 16);
-        const uint4 hdr = *reinterpret_cast<const uint4*>(slab + g.aux_off + ((uint64_t)(s / 8) * 64 + r) * 16);
-        float d1, m1;
-        q4k_scales(hdr, s % 8, d1, m1);
-        const uint32_t Q[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const uint32_t b = (Q[i] >> (8 * k)) & 0xFFu;
-                w[4 * i + k] = d1 * (float)(b & 15u) - m1;
-                w[16 + 4 * i + k] = d1 * (float)(b >> 4) - m1;
-            }
-    } else if constexpr (T == kQ5_K) {
-        const uint4 q = *reinterpret_cast<const uint4*>(slab + g.q_off + ((uint64_t)s * 64 + r) * 16);
-        const uint32_t qh = *reinterpret_cast<const uint32_t*>(slab + g.aux_off + ((uint64_t)s * 64 + r) * 4);
-        const uint4 hdr = *reinterpret_cast<const uint4*>(slab + g.sc_off + ((uint64_t)(s / 8) * 64 + r) * 16);
-        float d1, m1;
-        q4k_scales(hdr, s % 8, d1, m1);
-        const uint32_t Q[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t lo = (Q[i] & 0x0F0F0F0Fu) | ((qh << (4 - i)) & 0x10101010u);
-            const uint32_t hi = ((Q[i] >> 4) & 0x0F0F0F0Fu) | ((qh >> i) & 0x10101010u);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                w[4 * i + k] = d1 * ubyte(lo, k) - m1;
-                w[16 + 4 * i + k] = d1 * ubyte(hi, k) - m1;
-            }
-        }
-    } else if constexpr (T == kIQ4_XS) {
-        const uint4 q = *reinterpret_cast<const uint4*>(slab + g.q_off + ((uint64_t)s * 64 + r) * 16);
-        const uint2 hdr = *reinterpret_cast<const uint2*>(slab + g.aux_off + ((uint64_t)(s / 8) * 64 + r) * 8);
-        const float dl = h2f((uint16_t)(hdr.x & 0xFFFFu)) * (float)iq4xs_ls(hdr.x >> 16, hdr.y, s % 8);
-        const uint32_t Q[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t lo = iq4_lookup4(Q[i]), hi = iq4_lookup4(Q[i] >> 4);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                w[4 * i + k] = dl * (ubyte(lo, k) - 128.0f);
-                w[16 + 4 * i + k] = dl * (ubyte(hi, k) - 128.0f);
-            }
-        }
-    } else {  // Q6_K
-        const uint4 ql = *reinterpret_cast<const uint4*>(slab + g.q_off + ((uint64_t)s * 64 + r) * 16);
-        const uint2 qh = *reinterpret_cast<const uint2*>(slab + g.aux_off + ((uint64_t)s * 64 + r) * 8);
-        const uint32_t sb = s / 8, j = s % 8;
-        const uint8_t* scp = slab + g.sc_off + ((uint64_t)sb * 64 + r) * 16;
-        const float d = h2f(*reinterpret_cast<const uint16_t*>(slab + g.d_off + ((uint64_t)sb * 64 + r) * 2));
-        const float dA = d * (float)(int8_t)scp[2 * j], dB = d * (float)(int8_t)scp[2 * j + 1];
-        uint32_t lo[4], hi[4];
-        q6_slot_bytes(ql, qh, lo, hi);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                w[4 * i + k] = dA * (float)((int)((lo[i] >> (8 * k)) & 0xFFu) - 32);
-                w[16 + 4 * i + k] = dB * (float)((int)((hi[i] >> (8 * k)) & 0xFFu) - 32);
-            }
+        for (uint32_t k = 0; k < 4; ++k)
+            if (k < left) o[i + k] = w[k];
     }
 }
 
 template <uint32_t T>
-__global__ void k_dequant_slab(const uint8_t* __restrict__ w, uint32_t cols, uint32_t first_row, uint32_t n_rows,
-                               float* __restrict__ out, uint64_t out_stride, const int32_t* __restrict__ ids,
-                               uint32_t table_rows, uint32_t* status) {
-    const SlabGeom g = slab_geom(T, cols);
-    const uint32_t S = cols / kSlot;
-    const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (uint64_t)n_rows * S) return;
-    const uint32_t s = (uint32_t)(idx % S);
+__global__ __launch_bounds__(kDqThreads) void k_dequant_gguf(const uint8_t* __restrict__ w, uint64_t w_stride, uint32_t cols,
+                                                             uint32_t first_row, uint32_t blocks_per_row,
+                                                             float* __restrict__ out, uint64_t out_stride,
+                                                             const int32_t* __restrict__ ids, uint32_t table_rows,
+                                                             uint32_t* status) {
+    const uint32_t r = blockIdx.x / blocks_per_row;
+    const uint32_t i = (blockIdx.x % blocks_per_row) * kDqElems + 4 * threadIdx.x;
+    if (i >= cols) return;
     uint64_t row;
-    if (!table_row(ids, table_rows, first_row, idx / S, s == 0, status, row)) return;
-    float wv[32];
-    slab_slot_weights<T>(w + (row / kSlabRows) * g.slab_bytes, g, (uint32_t)(row % kSlabRows), s, wv);
-    float* o = out + (idx / S) * out_stride + (uint64_t)s * 32;
-    for (int i = 0; i < 32; ++i) o[i] = wv[i];
+    if (!table_row(ids, table_rows, first_row, r, i == 0, status, row)) return;
+    const uint8_t* p = w + row * w_stride;
+    float v[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) v[k] = i + k < cols ? gguf_elem<T>(p, i + k) : 0.0f;
+    store4(out + r * out_stride, i, cols - i, v);
+}
+
+// Exact fp32 weights 4 k .. 4 k + 3 of slot s of the row at lane r of `slab` (the reference's
+// expressions). Dword i = k % 4 of the slot's code record holds them, in the low nibbles (k < 4) or
+// the high ones.
+template <uint32_t T>
+__device__ __forceinline__ void slab_quad_weights(const uint8_t* __restrict__ slab, const SlabGeom& g, uint32_t r,
+                                                  uint32_t s, uint32_t k, float w[4]) {
+#pragma clang fp contract(off)
+    const uint32_t i = k & 3u, high = k >> 2;
+    const uint64_t sr = (uint64_t)s * 64 + r, br = (uint64_t)(s / 8) * 64 + r;
+    auto word = [&](uint64_t off) __attribute__((always_inline)) { return *reinterpret_cast<const uint32_t*>(slab + off); };
+    auto half = [&](uint64_t off) __attribute__((always_inline)) { return h2f(*reinterpret_cast<const uint16_t*>(slab + off)); };
+    if constexpr (T == kQ8_0) {
+        const float d = half(g.aux_off + sr * 2);
+        const uint32_t q = word(g.q_off + (((uint64_t)s * 2 + high) * 64 + r) * 16 + 4 * i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = sbyte(q, e) * d;
+        return;
+    }
+    const uint32_t q = word(g.q_off + sr * 16 + 4 * i);
+    const uint32_t nib = (high ? q >> 4 : q) & 0x0F0F0F0Fu;
+    if constexpr (T == kQ4_0) {
+        const float d = half(g.aux_off + sr * 2);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = (ubyte(nib, e) - 8.0f) * d;
+    } else if constexpr (T == kQ4_K || T == kQ5_K) {
+        const uint4 hdr = *reinterpret_cast<const uint4*>(slab + (T == kQ4_K ? g.aux_off : g.sc_off) + br * 16);
+        float d1, m1;
+        q4k_scales(hdr, s % 8, d1, m1);
+        uint32_t c = nib;
+        if constexpr (T == kQ5_K) {
+            const uint32_t qh = word(g.aux_off + sr * 4);
+            c |= (high ? qh >> i : qh << (4 - i)) & 0x10101010u;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = d1 * ubyte(c, e) - m1;
+    } else if constexpr (T == kIQ4_XS) {
+        const uint2 hdr = *reinterpret_cast<const uint2*>(slab + g.aux_off + br * 8);
+        const float dl = h2f((uint16_t)(hdr.x & 0xFFFFu)) * (float)iq4xs_ls(hdr.x >> 16, hdr.y, s % 8);
+        const uint32_t c = iq4_lookup4(nib);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = dl * (ubyte(c, e) - 128.0f);
+    } else {  // Q6_K: the top bits as q6_slot_bytes places them
+        const uint32_t h = word(g.aux_off + sr * 8 + 4 * (i >> 1));
+        const uint32_t top = (high ? ((i & 1u) ? h << 2 : h >> 2) : ((i & 1u) ? h << 4 : h)) & 0x30303030u;
+        const int8_t sc = *reinterpret_cast<const int8_t*>(slab + g.sc_off + br * 16 + 2 * (s % 8) + high);
+        const float dA = half(g.d_off + br * 2) * (float)sc;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = dA * (ubyte(nib | top, e) - 32.0f);
+    }
+}
+
+template <uint32_t T>
+__global__ __launch_bounds__(kDqThreads) void k_dequant_slab(const uint8_t* __restrict__ w, uint32_t cols, uint32_t first_row,
+                                                             uint32_t blocks_per_row, float* __restrict__ out,
+                                                             uint64_t out_stride, const int32_t* __restrict__ ids,
+                                                             uint32_t table_rows, uint32_t* status) {
+    const SlabGeom g = slab_geom(T, cols);
+    const uint32_t r = blockIdx.x / blocks_per_row;
+    const uint32_t i = (blockIdx.x % blocks_per_row) * kDqElems + 4 * threadIdx.x;
+    if (i >= cols) return;
+    uint64_t row;
+    if (!table_row(ids, table_rows, first_row, r, i == 0, status, row)) return;
+    float v[4];
+    slab_quad_weights<T>(w + (row / kSlabRows) * g.slab_bytes, g, (uint32_t)(row % kSlabRows), i / kSlot, i % kSlot / 4, v);
+    store4(out + r * out_stride, i, cols - i, v);
 }
 
 __global__ void k_fill_u32(uint32_t* p, uint64_t n, uint32_t v) {
@@ -274,12 +256,26 @@ int launch_unpack_slab(uint32_t type, const uint8_t* src, uint32_t rows, uint32_
     return hip_status(hipGetLastError(), "unpack_slab launch");
 }
 
+// Calls launch(grid, first table row, out, ids) for output rows [0, n_rows) in ranges whose blocks
+// fit one grid (`per` blocks per row).
+template <typename F>
+static int dequant_blocks(uint32_t n_rows, uint32_t per, uint32_t first_row, float* out, uint64_t out_stride,
+                          const int32_t* ids, F launch) {
+    const uint32_t most = std::max((1u << 23) / per, 1u);  // rows per launch (under 2^32 threads)
+    for (uint32_t r = 0; r < n_rows; r += std::min(most, n_rows - r)) {
+        const uint32_t n = std::min(most, n_rows - r);
+        if (int rc = launch(dim3(n * per), first_row + r, out + (uint64_t)r * out_stride, ids ? ids + r : nullptr)) return rc;
+    }
+    return HALO_MI_OK;
+}
+
 int launch_dequant_gguf(uint32_t type, const uint8_t* w, uint64_t w_stride, uint32_t cols, uint32_t first_row,
                         uint32_t n_rows, float* out, uint64_t out_stride, hipStream_t st, const int32_t* ids,
                         uint32_t table_rows, uint32_t* status) {
-    const uint64_t n = (uint64_t)n_rows * cols;
-    const dim3 grid((uint32_t)((n + 255) / 256)), block(256);
-#define HALO_MI_DQ(T) case T: hipLaunchKernelGGL(k_dequant_gguf<T>, grid, block, 0, st, w, w_stride, cols, first_row, n_rows, out, out_stride, ids, table_rows, status); break
+    const uint32_t per = (cols - 1) / kDqElems + 1;
+    const dim3 block(kDqThreads);
+#define HALO_MI_DQ(T) case T: hipLaunchKernelGGL(k_dequant_gguf<T>, grid, block, 0, st, w, w_stride, cols, first, per, o, out_stride, id, table_rows, status); break
+    return dequant_blocks(n_rows, per, first_row, out, out_stride, ids, [&](dim3 grid, uint32_t first, float* o, const int32_t* id) {
     switch (type) {
         HALO_MI_DQ(kF32);
         HALO_MI_DQ(kF16);
@@ -299,15 +295,17 @@ int launch_dequant_gguf(uint32_t type, const uint8_t* w, uint64_t w_stride, uint
         HALO_MI_DQ(kIQ4_XS);
         default: return set_error(HALO_MI_E_UNSUPPORTED, "dequant: type %u has no decoder", type);
     }
-#undef HALO_MI_DQ
     return hip_status(hipGetLastError(), "dequant_gguf launch");
+    });
+#undef HALO_MI_DQ
 }
 
 int launch_dequant_slab(uint32_t type, const uint8_t* w, uint32_t cols, uint32_t first_row, uint32_t n_rows, float* out,
                         uint64_t out_stride, hipStream_t st, const int32_t* ids, uint32_t table_rows, uint32_t* status) {
-    const uint64_t n = (uint64_t)n_rows * (cols / kSlot);
-    const dim3 grid((uint32_t)((n + 255) / 256)), block(256);
-#define HALO_MI_DQ(T) hipLaunchKernelGGL(k_dequant_slab<T>, grid, block, 0, st, w, cols, first_row, n_rows, out, out_stride, ids, table_rows, status)
+    const uint32_t per = (cols - 1) / kDqElems + 1;
+    const dim3 block(kDqThreads);
+#define HALO_MI_DQ(T) hipLaunchKernelGGL(k_dequant_slab<T>, grid, block, 0, st, w, cols, first, per, o, out_stride, id, table_rows, status)
+    return dequant_blocks(n_rows, per, first_row, out, out_stride, ids, [&](dim3 grid, uint32_t first, float* o, const int32_t* id) {
     switch (type) {
         case kQ4_0: HALO_MI_DQ(kQ4_0); break;
         case kQ8_0: HALO_MI_DQ(kQ8_0); break;
@@ -316,8 +314,9 @@ int launch_dequant_slab(uint32_t type, const uint8_t* w, uint32_t cols, uint32_t
         case kIQ4_XS: HALO_MI_DQ(kIQ4_XS); break;
         default: HALO_MI_DQ(kQ6_K); break;
     }
-#undef HALO_MI_DQ
     return hip_status(hipGetLastError(), "dequant_slab launch");
+    });
+#undef HALO_MI_DQ
 }
 
 int launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t st) {
