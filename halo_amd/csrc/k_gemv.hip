@@ -221,7 +221,13 @@ int launch_gemv_slab_t(GemvSlabArgs a, uint32_t slabs, Workspace* ws, uint64_t s
 template <uint32_t T>
 bool norm_in_kernel_t(uint32_t slabs, uint32_t cols, uint32_t mats, bool have_ws) {
     const EvenSplit ev = pick_even<T>(slabs, cols / kSlot, mats, have_ws);
-    const uint32_t nw = ev.W ? ev.nu : pick_split<T>(slabs, cols / kSlot, mats, have_ws).nw;
+    const GemvSplit sp = pick_split<T>(slabs, cols / kSlot, mats, have_ws);
+    // Without split K nothing is published, and every workgroup would run the chains: with more
+    // workgroups than CUs that is paid once per round of them. The RMS_NORM kernel first then costs
+    // one launch (Q6_K 248320 x 5120 with its logits, MI355X: 247.6 -> 195.1 us). Few workgroups, or a call with
+    // no workspace to normalize into, keep the norm inside.
+    if (!ev.W && sp.ks * mats == 1 && slabs > 256 && have_ws) return false;
+    const uint32_t nw = ev.W ? ev.nu : sp.nw;
     const size_t lds = ev.W ? even_lds_bytes<1>(ev.nu, nw) : mx_lds_bytes<1>(nw);
     const uint32_t full = cols - cols % 8u;
     return full > 0 && cols <= kNormMaxCols && cols % 32 == 0 && full <= kNormPerThread * 64 * nw &&
