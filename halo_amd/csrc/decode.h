@@ -80,12 +80,15 @@ __device__ __forceinline__ int iq4xs_ls(uint32_t sh, uint32_t sl, uint32_t j) {
     return (int)(((sl >> (4 * j)) & 15u) | (((sh >> (2 * j)) & 3u) << 4)) - 32;
 }
 // Four 4-bit codes in the low nibbles of q's bytes (the high nibbles are ignored) -> the
-// table's biased values (kIq4TabB) as bytes: a byte-permute over each table half with the
-// code's low 3 bits, then a third one that takes byte k from the half that bit 3 names.
+// table's values as bytes (BIASED: kIq4TabB, else the signed ones): a byte-permute over each
+// table half with the code's low 3 bits, then a third one that takes byte k from the half that bit
+// 3 names.
+template <bool BIASED = true>
 __device__ __forceinline__ uint32_t iq4_lookup4(uint32_t q) {
+    const uint32_t* tab = BIASED ? kIq4TabB : kIq4Tab;
     const uint32_t sel = q & 0x07070707u;
-    const uint32_t lo = __builtin_amdgcn_perm(kIq4TabB[1], kIq4TabB[0], sel);
-    const uint32_t hi = __builtin_amdgcn_perm(kIq4TabB[3], kIq4TabB[2], sel);
+    const uint32_t lo = __builtin_amdgcn_perm(tab[1], tab[0], sel);
+    const uint32_t hi = __builtin_amdgcn_perm(tab[3], tab[2], sel);
     return __builtin_amdgcn_perm(hi, lo, ((q >> 1) & 0x04040404u) | 0x03020100u);
 }
 

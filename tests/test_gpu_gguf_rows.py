@@ -64,3 +64,11 @@ def test_infinities_and_nan(hl, oracle, dev, t):
     assert isclose_bits(y[0], ref[0])
     assert np.array_equal(np.isnan(y), np.isnan(ref))
     assert np.array_equal(y[~np.isnan(ref)], ref[~np.isnan(ref)])
+
+
+@pytest.mark.parametrize("t", GGUF_TYPES)
+@pytest.mark.parametrize("rows,cols", [(1, 256), (8, 512), (17, 768), (9, 4608), (6144, 256), (6145, 256)])
+def test_one_vector_rounds(hl, oracle, dev, t, rows, cols):
+    """One vector with the products made ahead (up to 6144 rows): fewer chunks than producers, an odd last
+    round, more rounds than are loaded ahead, and the rows on either side of the rule."""
+    check(hl, oracle, dev, t, rows, cols, 1)
