@@ -19,64 +19,249 @@ using namespace dev;
 // Repack / unpack / dequantize
 // ==========================================================================================
 
-// One thread per (slab, block, row), row fastest: the 64 threads of a (slab, block) write each
-// of the block's slot records as one contiguous 1 KB, and each reads its row's block.
-__global__ void k_repack_slab(uint32_t type, const uint8_t* __restrict__ src, uint64_t src_stride, uint32_t rows,
-                              uint32_t cols, uint8_t* __restrict__ dst) {
-    const SlabGeom g = slab_geom(type, cols);
-    const uint32_t nblk = cols / block_elems(type), S = cols / kSlot;
-    const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint64_t slabs = (rows + kSlabRows - 1) / kSlabRows;
-    if (idx >= slabs * nblk * kSlabRows) return;
-    const uint32_t r = (uint32_t)(idx % kSlabRows);
-    const uint64_t sb = idx / kSlabRows;
-    const uint32_t b = (uint32_t)(sb % nblk);
-    const uint64_t slab = sb / nblk, row = slab * kSlabRows + r;
-    uint8_t* out = dst + slab * g.slab_bytes;
-    const uint8_t* s = src + row * src_stride + (uint64_t)b * block_bytes(type);
-    if (type == kQ4_K && ((reinterpret_cast<uintptr_t>(s) | src_stride) % 16) == 0) {
-        // vector path: 9 x 16 B in; 8 slot records and the header out as 16-byte stores
-        uint4 blk[9];
-#pragma unroll
-        for (int i = 0; i < 9; ++i) blk[i] = row < rows ? reinterpret_cast<const uint4*>(s)[i] : uint4{0, 0, 0, 0};
-        *reinterpret_cast<uint4*>(out + g.aux_off + ((uint64_t)b * 64 + r) * 16) = blk[0];
-#pragma unroll
-        for (int grp = 0; grp < 4; ++grp) {  // 32 quant bytes: sub-blocks 2 grp (low nibbles), 2 grp + 1 (high)
-            const uint4 A = blk[1 + 2 * grp], B = blk[2 + 2 * grp];
-            const uint32_t a[4] = {A.x, A.y, A.z, A.w}, c[4] = {B.x, B.y, B.z, B.w};
-            uint32_t lo[4], hi[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                lo[k] = (a[k] & 0x0F0F0F0Fu) | ((c[k] & 0x0F0F0F0Fu) << 4);
-                hi[k] = ((a[k] >> 4) & 0x0F0F0F0Fu) | (c[k] & 0xF0F0F0F0u);
-            }
-            *reinterpret_cast<uint4*>(out + g.q_off + (((uint64_t)b * 8 + 2 * grp) * 64 + r) * 16) = uint4{lo[0], lo[1], lo[2], lo[3]};
-            *reinterpret_cast<uint4*>(out + g.q_off + (((uint64_t)b * 8 + 2 * grp + 1) * 64 + r) * 16) = uint4{hi[0], hi[1], hi[2], hi[3]};
-        }
-        return;
-    }
-    uint8_t blk[210];
-    const uint32_t bb = block_bytes(type);
-    if (row < rows) {
-        for (uint32_t i = 0; i < bb; ++i) blk[i] = s[i];
-    } else {
-        for (uint32_t i = 0; i < bb; ++i) blk[i] = 0;
-    }
-    slab_pack_block(type, blk, out, g, S, r, b);
+// One thread per (slab, kRepackBlocks consecutive blocks, row), row fastest: the 64 threads of a
+// (slab, block) read or write each of the block's slot records as one contiguous 1 KB, and each
+// works on its own row's block with 16-byte accesses at whatever alignment the row has, all in
+// registers. Bound by HBM: the rows' accesses are one line apart per lane, and a thread of a
+// 32-weight format takes several blocks so that it uses most of a line at once. Measured on MI355X,
+// 17408 x 5120, repack / unpack us (bytes moved one by one through a block in scratch memory, and
+// unpack with the blocks of a row side by side, before): Q4_0 61 / 125 -> 37 / 58, Q8_0 121 / 304 ->
+// 52 / 70, Q4_K 23 (its own 16-byte path) / 589 -> 23 / 26, Q5_K 179 / 738 -> 29 / 30, Q6_K 217 / 886
+// -> 39 / 42 (73 MB: 3.7 TB/s read and written), IQ4_XS 139 / 609 -> 25 / 25.
+template <uint32_t T>
+constexpr uint32_t kRepackBlocks = T == kQ4_0 ? 8u : T == kQ8_0 ? 4u : 1u;
+
+__device__ __forceinline__ uint4 ld16(const uint8_t* p) {
+    uint4 v;
+    __builtin_memcpy(&v, p, 16);
+    return v;
+}
+__device__ __forceinline__ void st16(uint8_t* p, const uint4& v) { __builtin_memcpy(p, &v, 16); }
+__device__ __forceinline__ void unwords(const uint4& v, uint32_t w[4]) {
+    w[0] = v.x;
+    w[1] = v.y;
+    w[2] = v.z;
+    w[3] = v.w;
 }
 
-__global__ void k_unpack_slab(uint32_t type, const uint8_t* __restrict__ src, uint32_t rows, uint32_t cols,
-                              uint8_t* __restrict__ dst, uint64_t dst_stride) {
-    const SlabGeom g = slab_geom(type, cols);
-    const uint32_t nblk = cols / block_elems(type), S = cols / kSlot;
+// The two slot records of 32 bytes holding 64 4-bit codes (a: bytes 0..15, c: 16..31): the low
+// nibbles' slot, then the high nibbles'; and back.
+__device__ __forceinline__ void nibbles_to_slots(const uint4& a4, const uint4& c4, uint4& lo, uint4& hi) {
+    uint32_t a[4], c[4], l[4], h[4];
+    unwords(a4, a);
+    unwords(c4, c);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        l[k] = (a[k] & 0x0F0F0F0Fu) | ((c[k] & 0x0F0F0F0Fu) << 4);
+        h[k] = ((a[k] >> 4) & 0x0F0F0F0Fu) | (c[k] & 0xF0F0F0F0u);
+    }
+    lo = uint4{l[0], l[1], l[2], l[3]};
+    hi = uint4{h[0], h[1], h[2], h[3]};
+}
+// (the map is its own inverse: lo, hi -> a, c)
+
+template <uint32_t T>
+__device__ __forceinline__ void repack_block(const uint8_t* __restrict__ s, bool live, uint8_t* __restrict__ out, const SlabGeom& g,
+                                             uint32_t r, uint32_t b) {
+    auto in = [&](uint32_t o) __attribute__((always_inline)) { return live ? ld16(s + o) : uint4{0, 0, 0, 0}; };
+    auto in2 = [&](uint32_t o) __attribute__((always_inline)) {
+        uint16_t v = 0;
+        if (live) __builtin_memcpy(&v, s + o, 2);
+        return v;
+    };
+    auto rec = [&](uint64_t off, uint64_t i, uint32_t bytes) __attribute__((always_inline)) { return out + off + (i * 64 + r) * bytes; };
+    if constexpr (T == kQ4_0 || T == kQ8_0) {
+        const uint16_t d = in2(0);
+        const uint4 q = in(2);
+        if constexpr (T == kQ4_0) {
+            *reinterpret_cast<uint4*>(rec(g.q_off, b, 16)) = q;
+        } else {
+            const uint4 q1 = in(18);
+            *reinterpret_cast<uint4*>(rec(g.q_off, 2 * (uint64_t)b, 16)) = q;
+            *reinterpret_cast<uint4*>(rec(g.q_off, 2 * (uint64_t)b + 1, 16)) = q1;
+        }
+        *reinterpret_cast<uint16_t*>(rec(g.aux_off, b, 2)) = d;
+    } else if constexpr (T == kIQ4_XS) {
+        uint2 hdr{0, 0};
+        if (live) __builtin_memcpy(&hdr, s, 8);
+        uint4 q[8];
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) q[j] = in(8 + 16 * j);
+        *reinterpret_cast<uint2*>(rec(g.aux_off, b, 8)) = hdr;
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) *reinterpret_cast<uint4*>(rec(g.q_off, (uint64_t)b * 8 + j, 16)) = q[j];
+    } else if constexpr (T == kQ4_K || T == kQ5_K) {
+        constexpr uint32_t Q = T == kQ4_K ? 16 : 48;
+        const uint4 hdr = in(0);
+        uint4 q[8], qh[2];
+#pragma unroll
+        for (uint32_t i = 0; i < 8; ++i) q[i] = in(Q + 16 * i);
+        if constexpr (T == kQ5_K) {
+            qh[0] = in(16);
+            qh[1] = in(32);
+        }
+        *reinterpret_cast<uint4*>(rec(T == kQ4_K ? g.aux_off : g.sc_off, b, 16)) = hdr;
+#pragma unroll
+        for (uint32_t grp = 0; grp < 4; ++grp) {  // sub-blocks 2 grp (low nibbles), 2 grp + 1 (high)
+            uint4 lo, hi;
+            nibbles_to_slots(q[2 * grp], q[2 * grp + 1], lo, hi);
+            *reinterpret_cast<uint4*>(rec(g.q_off, (uint64_t)b * 8 + 2 * grp, 16)) = lo;
+            *reinterpret_cast<uint4*>(rec(g.q_off, (uint64_t)b * 8 + 2 * grp + 1, 16)) = hi;
+        }
+        if constexpr (T == kQ5_K) {  // bit j of qh dword i -> bit i of the bytes of slot j's word
+            uint32_t h[8];
+            unwords(qh[0], h);
+            unwords(qh[1], h + 4);
+#pragma unroll
+            for (uint32_t j = 0; j < 8; ++j) {
+                uint32_t w = 0;
+#pragma unroll
+                for (uint32_t i = 0; i < 8; ++i) w |= ((h[i] >> j) & 0x01010101u) << i;
+                *reinterpret_cast<uint32_t*>(rec(g.aux_off, (uint64_t)b * 8 + j, 4)) = w;
+            }
+        }
+    } else {  // Q6_K
+        uint4 q[8], qh[4];
+#pragma unroll
+        for (uint32_t i = 0; i < 8; ++i) q[i] = in(16 * i);
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) qh[i] = in(128 + 16 * i);
+        const uint4 sc = in(192);
+        const uint16_t d = in2(208);
+        *reinterpret_cast<uint4*>(rec(g.sc_off, b, 16)) = sc;
+        *reinterpret_cast<uint16_t*>(rec(g.d_off, b, 2)) = d;
+#pragma unroll
+        for (uint32_t n = 0; n < 2; ++n) {
+            // 32 code bytes 64 n + 32 p: slots 4 n + p (low nibbles) and 4 n + 2 + p (high)
+#pragma unroll
+            for (uint32_t p = 0; p < 2; ++p) {
+                uint4 lo, hi;
+                nibbles_to_slots(q[4 * n + 2 * p], q[4 * n + 2 * p + 1], lo, hi);
+                *reinterpret_cast<uint4*>(rec(g.q_off, (uint64_t)b * 8 + 4 * n + p, 16)) = lo;
+                *reinterpret_cast<uint4*>(rec(g.q_off, (uint64_t)b * 8 + 4 * n + 2 + p, 16)) = hi;
+            }
+            uint32_t h[8];
+            unwords(qh[2 * n], h);
+            unwords(qh[2 * n + 1], h + 4);
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k) {  // slot 4 n + k: bits 2 k .. 2 k + 1 (q6_qh_byte's places)
+                uint32_t w[2];
+#pragma unroll
+                for (uint32_t i = 0; i < 2; ++i) {
+                    auto t = [&](uint32_t x) __attribute__((always_inline)) { return (h[x] >> (2 * k)) & 0x03030303u; };
+                    w[i] = t(2 * i + 1) | (t(2 * i + 5) << 2) | (t(2 * i) << 4) | (t(2 * i + 4) << 6);
+                }
+                *reinterpret_cast<uint2*>(rec(g.aux_off, (uint64_t)b * 8 + 4 * n + k, 8)) = uint2{w[0], w[1]};
+            }
+        }
+    }
+}
+
+// repack_block's inverse: the block's GGUF bytes at d.
+template <uint32_t T>
+__device__ __forceinline__ void unpack_block(const uint8_t* __restrict__ src, uint8_t* __restrict__ d, const SlabGeom& g, uint32_t r,
+                                             uint32_t b) {
+    auto rec = [&](uint64_t off, uint64_t i, uint32_t bytes) __attribute__((always_inline)) { return src + off + (i * 64 + r) * bytes; };
+    auto q = [&](uint64_t i) __attribute__((always_inline)) { return *reinterpret_cast<const uint4*>(rec(g.q_off, i, 16)); };
+    if constexpr (T == kQ4_0 || T == kQ8_0) {
+        __builtin_memcpy(d, rec(g.aux_off, b, 2), 2);
+        if constexpr (T == kQ4_0) {
+            st16(d + 2, q(b));
+        } else {
+            st16(d + 2, q(2 * (uint64_t)b));
+            st16(d + 18, q(2 * (uint64_t)b + 1));
+        }
+    } else if constexpr (T == kIQ4_XS) {
+        const uint2 hdr = *reinterpret_cast<const uint2*>(rec(g.aux_off, b, 8));
+        __builtin_memcpy(d, &hdr, 8);
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) st16(d + 8 + 16 * j, q((uint64_t)b * 8 + j));
+    } else if constexpr (T == kQ4_K || T == kQ5_K) {
+        constexpr uint32_t Q = T == kQ4_K ? 16 : 48;
+        st16(d, *reinterpret_cast<const uint4*>(rec(T == kQ4_K ? g.aux_off : g.sc_off, b, 16)));
+        if constexpr (T == kQ5_K) {
+            uint32_t h[8] = {};
+#pragma unroll
+            for (uint32_t j = 0; j < 8; ++j) {
+                const uint32_t w = *reinterpret_cast<const uint32_t*>(rec(g.aux_off, (uint64_t)b * 8 + j, 4));
+#pragma unroll
+                for (uint32_t i = 0; i < 8; ++i) h[i] |= ((w >> i) & 0x01010101u) << j;
+            }
+            st16(d + 16, uint4{h[0], h[1], h[2], h[3]});
+            st16(d + 32, uint4{h[4], h[5], h[6], h[7]});
+        }
+#pragma unroll
+        for (uint32_t grp = 0; grp < 4; ++grp) {
+            uint4 a, c;
+            nibbles_to_slots(q((uint64_t)b * 8 + 2 * grp), q((uint64_t)b * 8 + 2 * grp + 1), a, c);
+            st16(d + Q + 32 * grp, a);
+            st16(d + Q + 32 * grp + 16, c);
+        }
+    } else {  // Q6_K
+#pragma unroll
+        for (uint32_t n = 0; n < 2; ++n) {
+#pragma unroll
+            for (uint32_t p = 0; p < 2; ++p) {
+                uint4 a, c;
+                nibbles_to_slots(q((uint64_t)b * 8 + 4 * n + p), q((uint64_t)b * 8 + 4 * n + 2 + p), a, c);
+                st16(d + 64 * n + 32 * p, a);
+                st16(d + 64 * n + 32 * p + 16, c);
+            }
+            uint32_t h[8] = {};
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k) {
+                const uint2 w2 = *reinterpret_cast<const uint2*>(rec(g.aux_off, (uint64_t)b * 8 + 4 * n + k, 8));
+                const uint32_t w[2] = {w2.x, w2.y};
+#pragma unroll
+                for (uint32_t i = 0; i < 2; ++i) {
+                    h[2 * i + 1] |= (w[i] & 0x03030303u) << (2 * k);
+                    h[2 * i + 5] |= ((w[i] >> 2) & 0x03030303u) << (2 * k);
+                    h[2 * i] |= ((w[i] >> 4) & 0x03030303u) << (2 * k);
+                    h[2 * i + 4] |= ((w[i] >> 6) & 0x03030303u) << (2 * k);
+                }
+            }
+            st16(d + 128 + 32 * n, uint4{h[0], h[1], h[2], h[3]});
+            st16(d + 128 + 32 * n + 16, uint4{h[4], h[5], h[6], h[7]});
+        }
+        st16(d + 192, *reinterpret_cast<const uint4*>(rec(g.sc_off, b, 16)));
+        __builtin_memcpy(d + 208, rec(g.d_off, b, 2), 2);
+    }
+}
+
+template <uint32_t T>
+__global__ __launch_bounds__(256) void k_repack_slab(const uint8_t* __restrict__ src, uint64_t src_stride, uint32_t rows, uint32_t cols,
+                                                     uint8_t* __restrict__ dst) {
+    constexpr uint32_t NB = kRepackBlocks<T>;
+    const SlabGeom g = slab_geom(T, cols);
+    const uint32_t nblk = cols / block_elems(T), groups = (nblk + NB - 1) / NB;
     const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (uint64_t)rows * nblk) return;
-    const uint64_t row = idx / nblk;
-    const uint32_t b = (uint32_t)(idx % nblk);
-    uint8_t blk[210];
-    slab_unpack_block(type, src + (row / kSlabRows) * g.slab_bytes, blk, g, S, (uint32_t)(row % kSlabRows), b);
-    uint8_t* d = dst + row * dst_stride + (uint64_t)b * block_bytes(type);
-    for (uint32_t i = 0; i < block_bytes(type); ++i) d[i] = blk[i];
+    const uint32_t r = (uint32_t)(idx % kSlabRows);
+    const uint64_t slab = idx / kSlabRows / groups, row = slab * kSlabRows + r;
+    if (slab * kSlabRows >= rows) return;
+    const uint32_t b0 = (uint32_t)(idx / kSlabRows % groups) * NB;
+    const bool live = row < rows;
+#pragma unroll
+    for (uint32_t k = 0; k < NB; ++k)
+        if (b0 + k < nblk)
+            repack_block<T>(src + (live ? row : 0) * src_stride + (uint64_t)(b0 + k) * block_bytes(T), live, dst + slab * g.slab_bytes, g,
+                            r, b0 + k);
+}
+
+template <uint32_t T>
+__global__ __launch_bounds__(256) void k_unpack_slab(const uint8_t* __restrict__ src, uint32_t rows, uint32_t cols,
+                                                     uint8_t* __restrict__ dst, uint64_t dst_stride) {
+    constexpr uint32_t NB = kRepackBlocks<T>;
+    const SlabGeom g = slab_geom(T, cols);
+    const uint32_t nblk = cols / block_elems(T), groups = (nblk + NB - 1) / NB;
+    const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t r = (uint32_t)(idx % kSlabRows);
+    const uint64_t slab = idx / kSlabRows / groups, row = slab * kSlabRows + r;
+    if (row >= rows) return;
+    const uint32_t b0 = (uint32_t)(idx / kSlabRows % groups) * NB;
+#pragma unroll
+    for (uint32_t k = 0; k < NB; ++k)
+        if (b0 + k < nblk)
+            unpack_block<T>(src + slab * g.slab_bytes, dst + row * dst_stride + (uint64_t)(b0 + k) * block_bytes(T), g, r, b0 + k);
 }
 
 // The table row of output row r: first_row + r, or ids[r] (GET_ROWS). An id outside the table
@@ -240,19 +425,40 @@ int launch_stream_read(const void* p, uint64_t bytes, uint32_t workgroups, uint3
     return hip_status(hipGetLastError(), "stream_read launch");
 }
 
+// Threads of a repack or unpack launch: one per row (of whole slabs) and kRepackBlocks blocks
+template <uint32_t T>
+static dim3 repack_grid(uint32_t rows, uint32_t cols) {
+    const uint64_t groups = (cols / block_elems(T) + kRepackBlocks<T> - 1) / kRepackBlocks<T>;
+    return dim3((uint32_t)((((uint64_t)rows + kSlabRows - 1) / kSlabRows * kSlabRows * groups + 255) / 256));
+}
+
 int launch_repack_slab(uint32_t type, const uint8_t* src, uint64_t src_stride, uint32_t rows, uint32_t cols,
                        uint8_t* dst, hipStream_t st) {
-    const uint64_t n = (uint64_t)(rows + kSlabRows - 1) / kSlabRows * kSlabRows * (cols / block_elems(type));
-    hipLaunchKernelGGL(k_repack_slab, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, st, type, src, src_stride, rows,
-                       cols, dst);
+#define HALO_MI_RP(T) hipLaunchKernelGGL(k_repack_slab<T>, repack_grid<T>(rows, cols), dim3(256), 0, st, src, src_stride, rows, cols, dst)
+    switch (type) {
+        case kQ4_0: HALO_MI_RP(kQ4_0); break;
+        case kQ8_0: HALO_MI_RP(kQ8_0); break;
+        case kQ4_K: HALO_MI_RP(kQ4_K); break;
+        case kQ5_K: HALO_MI_RP(kQ5_K); break;
+        case kIQ4_XS: HALO_MI_RP(kIQ4_XS); break;
+        default: HALO_MI_RP(kQ6_K); break;
+    }
+#undef HALO_MI_RP
     return hip_status(hipGetLastError(), "repack_slab launch");
 }
 
 int launch_unpack_slab(uint32_t type, const uint8_t* src, uint32_t rows, uint32_t cols, uint8_t* dst,
                        uint64_t dst_stride, hipStream_t st) {
-    const uint64_t n = (uint64_t)rows * (cols / block_elems(type));
-    hipLaunchKernelGGL(k_unpack_slab, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, st, type, src, rows, cols, dst,
-                       dst_stride);
+#define HALO_MI_UP(T) hipLaunchKernelGGL(k_unpack_slab<T>, repack_grid<T>(rows, cols), dim3(256), 0, st, src, rows, cols, dst, dst_stride)
+    switch (type) {
+        case kQ4_0: HALO_MI_UP(kQ4_0); break;
+        case kQ8_0: HALO_MI_UP(kQ8_0); break;
+        case kQ4_K: HALO_MI_UP(kQ4_K); break;
+        case kQ5_K: HALO_MI_UP(kQ5_K); break;
+        case kIQ4_XS: HALO_MI_UP(kIQ4_XS); break;
+        default: HALO_MI_UP(kQ6_K); break;
+    }
+#undef HALO_MI_UP
     return hip_status(hipGetLastError(), "unpack_slab launch");
 }
 
