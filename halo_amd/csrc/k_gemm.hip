@@ -1274,9 +1274,12 @@ void launch_reduce(const GemmPcArgs& p, hipStream_t st) {
 }
 
 // Rows [m_start, m_start + mc) of x to bf16 fragments, zero-padded to m_pad rows; with the
-// fused norm, each row's 1 / rms first (k_rms_inv_rows into ws->inv).
+// fused norm in one launch (k_norm_to_frag), or for rows too wide for it each row's 1 / rms first
+// (k_rms_inv_rows into ws->inv).
 int stage_x(const GemmArgs& a, uint64_t m_start, uint32_t mc, uint32_t m_pad, Workspace* ws, hipStream_t st) {
     const float* x = a.x + m_start * a.x_stride;
+    if (a.norm_w && norm_to_frag_fits(a.cols))
+        return launch_norm_to_frag(x, a.x_stride, mc, m_pad, a.cols, a.norm_eps, a.norm_w, ws->xb, st);
     if (a.norm_w)
         if (int rc = launch_rms_inv(x, a.x_stride, mc, a.cols, a.norm_eps, ws->inv, st)) return rc;
     const uint64_t n8 = (uint64_t)m_pad * (a.cols / 8);

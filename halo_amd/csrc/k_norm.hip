@@ -108,6 +108,89 @@ __global__ __launch_bounds__(kNormBlock) void k_rms_inv_rows(const float* __rest
     if (threadIdx.x == 0) inv[blockIdx.x] = s;
 }
 
+// The GEMM's staged x with the fused norm: rows of x normalized as cpu::rms_norm rounds them,
+// (x * inv) * w, then to bf16 (RNE) in the A-fragment order of k_x_to_frag (k_gemm.hip): the 8
+// values of octet o (k = 8 o ..) of row m at 16-byte entry ((m / 32) * (cols / 16) + o / 2) * 64 +
+// 32 (o % 2) + m % 32; rows in [n_vec, m_pad) are zero. One launch in place of k_rms_inv_rows and
+// k_x_to_frag, with x read once.
+// A workgroup takes kFragRows rows: their chains run side by side in one wave, in the time of one
+// row's 8, and their entries of an octet are one 32-byte run. What bounds it is one round trip to
+// memory and the chains; the rows stay in registers meanwhile. Thread t has octets t / 2 + 256 i of
+// row t % 2. Measured on MI355X, what the norm adds to a Q4_K 5120 x 5120 GEMM at 13 / 64 / 200 / 512
+// rows of x: 5.4 / 5.8 / 6.0 / 6.9 us with the two launches, 3.0 / 3.0 / 2.4 / 3.4 here; 4 rows and
+// 1024 threads 4.9 / 4.9 / 4.4 / 3.2, one row and 256 threads 2.7 / 2.6 / 2.4 / 4.9.
+constexpr uint32_t kFragRows = 2, kFragBlock = 512, kFragOcts = kFragBlock / kFragRows;
+constexpr uint32_t kFragMaxCols = 8192;  // LDS for the squares of kFragRows rows
+// LDS floats of a row's squares; rows start 32 banks apart, so a wave's writes (32 octets of 2 rows) do not collide
+__host__ __device__ constexpr uint32_t frag_row_floats(uint32_t cols) {
+    return 8 * dev::norm_chain_stride(cols) + ((32 - 8 * dev::norm_chain_stride(cols)) & 63u);
+}
+
+template <uint32_t IT>
+__global__ __launch_bounds__(kFragBlock) void k_norm_to_frag(const float* __restrict__ x, uint64_t x_stride, uint32_t n_vec, uint32_t cols,
+                                                             float eps, const float* __restrict__ w, uint4* __restrict__ out) {
+#pragma clang fp contract(off)
+    extern __shared__ __align__(16) float lds[];
+    const uint32_t tid = threadIdx.x, row = tid % kFragRows, m = blockIdx.x * kFragRows + row, octs = cols / 8;
+    const uint32_t cs = dev::norm_chain_stride(cols), rs = frag_row_floats(cols);
+    const bool live = m < n_vec;
+    float v[IT][8], wv[IT][8];
+    auto load8 = [](const float* p, float (&d)[8]) __attribute__((always_inline)) {
+        const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);
+        d[0] = a.x;
+        d[1] = a.y;
+        d[2] = a.z;
+        d[3] = a.w;
+        d[4] = b.x;
+        d[5] = b.y;
+        d[6] = b.z;
+        d[7] = b.w;
+    };
+    if (blockIdx.x * kFragRows < n_vec) {  // (the whole workgroup: a block of padding rows only writes zeros)
+#pragma unroll
+        for (uint32_t i = 0; i < IT; ++i) {
+            const uint32_t o = min(tid / kFragRows + kFragOcts * i, octs - 1);  // past the end: not used
+            load8(x + (uint64_t)min(m, n_vec - 1) * x_stride + 8 * o, v[i]);
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < IT; ++i) {
+            const uint32_t o = tid / kFragRows + kFragOcts * i;
+#pragma unroll
+            for (uint32_t e = 0; e < 8; ++e)
+                if (o < octs) lds[row * rs + e * cs + o] = v[i][e] * v[i][e];
+        }
+        __syncthreads();
+        // the norm weights' elements, 4-byte loads (norm_w has no more alignment), while the chains run
+#pragma unroll
+        for (uint32_t i = 0; i < IT; ++i) {
+            const uint32_t o = min(tid / kFragRows + kFragOcts * i, octs - 1);
+#pragma unroll
+            for (uint32_t e = 0; e < 8; ++e) wv[i][e] = w[8 * o + e];
+        }
+        if (tid < 64) {
+            const uint32_t r = tid / 8 % kFragRows;  // (lanes 16 .. 63 repeat the rows)
+            const float p = dev::norm_chain_ahead(lds + r * rs + tid % 8 * cs, octs, 0.0f);
+            const float inv = dev::norm_finish(p, x, cols, cols, eps, tid % 8);
+            if (tid < 8 * kFragRows && tid % 8 == 0) lds[kFragRows * rs + r] = inv;
+        }
+        __syncthreads();
+    }
+    const float inv = live ? lds[kFragRows * rs + row] : 0.0f;
+#pragma unroll
+    for (uint32_t i = 0; i < IT; ++i) {
+        const uint32_t o = tid / kFragRows + kFragOcts * i;
+        dev::bf16x8 b{};
+        if (live) {
+#pragma unroll
+            for (uint32_t e = 0; e < 8; ++e) {
+                const float t = v[i][e] * inv;
+                b[e] = (__bf16)(t * wv[i][e]);
+            }
+        }
+        if (o < octs) out[((uint64_t)(m / 32) * (octs / 2) + o / 2) * 64 + 32 * (o % 2) + m % 32] = __builtin_bit_cast(uint4, b);
+    }
+}
+
 // Calls f(integral constant PT) with the least of 4, 8, 12, 16 loads per thread that cover a chunk of the row
 template <typename F>
 void with_loads(uint32_t cols, F f) {
@@ -127,6 +210,22 @@ int launch_rms_norm(const float* x, uint64_t x_stride, const float* w, float* ou
         hipLaunchKernelGGL(k_rms_norm_rows<pt()>, dim3(rows), dim3(kNormBlock), 0, st, x, x_stride, w, out, out_stride, cols, eps);
     });
     return hip_status(hipGetLastError(), "rms_norm launch");
+}
+
+bool norm_to_frag_fits(uint32_t cols) { return cols > 0 && cols <= kFragMaxCols && cols % 32 == 0; }
+
+int launch_norm_to_frag(const float* x, uint64_t x_stride, uint32_t n_vec, uint32_t m_pad, uint32_t cols, float eps, const float* w,
+                        __bf16* out, hipStream_t st) {
+    const size_t lds = (kFragRows * frag_row_floats(cols) + kFragRows) * sizeof(float);
+    const dim3 grid(m_pad / kFragRows), block(kFragBlock);
+    uint4* o = reinterpret_cast<uint4*>(out);
+    switch ((cols / 8 + kFragOcts - 1) / kFragOcts) {
+        case 1: hipLaunchKernelGGL(k_norm_to_frag<1>, grid, block, lds, st, x, x_stride, n_vec, cols, eps, w, o); break;
+        case 2: hipLaunchKernelGGL(k_norm_to_frag<2>, grid, block, lds, st, x, x_stride, n_vec, cols, eps, w, o); break;
+        case 3: hipLaunchKernelGGL(k_norm_to_frag<3>, grid, block, lds, st, x, x_stride, n_vec, cols, eps, w, o); break;
+        default: hipLaunchKernelGGL(k_norm_to_frag<4>, grid, block, lds, st, x, x_stride, n_vec, cols, eps, w, o); break;
+    }
+    return hip_status(hipGetLastError(), "norm staging launch");
 }
 
 int launch_rms_inv(const float* x, uint64_t x_stride, uint32_t rows, uint32_t cols, float eps, float* inv,

@@ -214,6 +214,11 @@ int launch_swiglu(const float* g, uint64_t gs, const float* u, uint64_t us, floa
 // of a normalized x.
 int launch_rms_norm(const float* x, uint64_t x_stride, const float* w, float* out, uint64_t out_stride, uint32_t rows,
                     uint32_t cols, float eps, hipStream_t st);
+// norm_to_frag: rows of x (16-byte aligned) normalized and staged as bf16 in the GEMM's A-fragment
+// order, zero-padded to m_pad rows (a multiple of 32), in one launch, for the cols that fit.
+bool norm_to_frag_fits(uint32_t cols);
+int launch_norm_to_frag(const float* x, uint64_t x_stride, uint32_t n_vec, uint32_t m_pad, uint32_t cols, float eps, const float* w,
+                        __bf16* out, hipStream_t st);
 int launch_rms_inv(const float* x, uint64_t x_stride, uint32_t rows, uint32_t cols, float eps, float* inv,
                    hipStream_t st);
 
