@@ -1481,6 +1481,13 @@ int launch_gemm_pc(uint32_t type, const GemmArgs& a, hipStream_t st) {
             // M = 64 57.3 -> 49.0 us, M = 128 70.4 -> 68.4, M = 256 105.2 -> 102.5, against 16)
             const uint32_t cap = main_units == 0 ? 16u : (MB == 1 ? 2u : 8u);
             kc = (uint32_t)std::min<uint64_t>({cus / std::max<uint64_t>(rest, 1), S / 8, cap});
+            // Every tile split, 64-row tiles: two workgroups fit a CU, and with both there one's stage
+            // barriers hide behind the other's work, as long as a chunk has at least 4 super-blocks
+            // (MI355X, M = 64, us at one and two workgroups per CU: Q5_K 12288 x 5120 34.8 -> 31.5 with 5
+            // chunks, Q6_K 5120 x 17408 41.5 -> 38.2 with 12; with 2 super-blocks per chunk Q5_K 5120 x
+            // 6144 23.3 -> 25.4, Q4_K 6144 x 5120 21.5 -> 24.1). 128- and 256-row tiles measured slower.
+            if (main_units == 0 && MB == 1)
+                kc = std::max(kc, (uint32_t)std::min<uint64_t>({2 * cus / std::max<uint64_t>(rest, 1), S / 32, cap}));
             while (kc > 1 && rest * kc * BM * kPcW > kPartialFloats) --kc;
             if (kc < 2) main_units = units;  // nothing to gain: one launch
         }

@@ -1,0 +1,32 @@
+"""The bf16 GEMM on 64-row tiles whose matrix is split over K for two workgroups per CU: around the tile counts
+and widths where the chunk count changes, against the fp64 product of the bf16-rounded operands within the
+GEMM's accumulation bound."""
+import numpy as np
+import pytest
+
+from helpers import Q4_K, Q6_K, gemm_emulated, make_weights
+from test_gpu_parity import host, say, to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q6_K])
+# 33 / 3 / 12 tiles of 128 rows; 4, 8, 9 and 17 super-blocks of K
+@pytest.mark.parametrize("rows,cols", [(4200, 1024), (300, 2048), (1500, 2304), (1472, 4352)])
+@pytest.mark.parametrize("n_vec", [33, 64])
+def test_split_for_two_workgroups(hl, oracle, dev, t, rows, cols, n_vec):
+    import torch
+
+    say("two per CU", t, rows, cols, n_vec)
+    buf, _ = make_weights(t, rows, cols, seed=rows + cols)
+    x = np.random.default_rng(n_vec).normal(0, 1, (n_vec, cols)).astype(np.float32)
+    wq = to_dev(buf, dev)
+    slab = torch.empty(hl.slab_bytes(t, rows, cols), dtype=torch.uint8, device=dev)
+    hl.repack_slab(t, wq, rows, cols, slab)
+    y = torch.full((n_vec, rows), float("nan"), dtype=torch.float32, device=dev)
+    xd = to_dev(x, dev)
+    hl.gemv(t, slab, xd, y, rows, cols, n_vec, variant=3)
+    got = host(y)
+    size = rows * cols // 256 * (144 if t == Q4_K else 210)
+    ref, tol = gemm_emulated(oracle, t, buf[:size], rows, cols, x)
+    assert np.all(np.abs(got - ref) <= tol)
