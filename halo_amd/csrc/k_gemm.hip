@@ -1467,11 +1467,16 @@ int launch_gemm_pc(uint32_t type, const GemmArgs& a, hipStream_t st) {
         const uint32_t m_tiles = (mc + BM - 1) / BM;
         if (int rc = stage_x(a, m_start, mc, m_tiles * BM, ws, st)) return rc;
         float* y = a.y + m_start * a.y_stride;
-        // whole rounds of tiles, then the rest split over K; a matrix whose tiles cannot fill
-        // half the chip is split over K altogether
+        // whole rounds of tiles, then the rest split over K; a matrix whose tiles fill at most half
+        // the chip is split over K altogether, and on 64-row tiles so is one of less than a whole round
+        // that has two chunks or more to fill two workgroups per CU with (MI355X, Q4_K gate/up pairs
+        // of 5120 columns, M = 64, us whole and split: 128 units 46 -> 32 with 4 chunks, 160 47 -> 38
+        // with 3, 224 50 -> 45 and 255 49 -> 47 with 2; M = 128 / 256: 128 units 50 / 64 -> 41 / 54,
+        // 160 and more no faster; 256 units at M = 64 44 -> 46)
         const uint64_t tiles = (uint64_t)units * m_tiles;
         uint32_t main_units = units, kc = 1;
-        if (S % 8 == 0 && ((tiles > cus && tiles % cus != 0) || 2 * tiles < cus)) {
+        const uint32_t two_kc = (uint32_t)std::min<uint64_t>({2 * cus / std::max<uint64_t>(tiles, 1), S / 32, 16});
+        if (S % 8 == 0 && ((tiles > cus && tiles % cus != 0) || 2 * tiles <= cus || (MB == 1 && tiles < cus && two_kc >= 2))) {
             main_units = tiles > cus ? (uint32_t)(tiles / cus * cus / m_tiles) : 0u;
             const uint64_t rest = (uint64_t)(units - main_units) * m_tiles;
             // Tiles left over beside a whole round: 64-row tiles run two workgroups per CU, so
@@ -1486,8 +1491,7 @@ int launch_gemm_pc(uint32_t type, const GemmArgs& a, hipStream_t st) {
             // (MI355X, M = 64, us at one and two workgroups per CU: Q5_K 12288 x 5120 34.8 -> 31.5 with 5
             // chunks, Q6_K 5120 x 17408 41.5 -> 38.2 with 12; with 2 super-blocks per chunk Q5_K 5120 x
             // 6144 23.3 -> 25.4, Q4_K 6144 x 5120 21.5 -> 24.1). 128- and 256-row tiles measured slower.
-            if (main_units == 0 && MB == 1)
-                kc = std::max(kc, (uint32_t)std::min<uint64_t>({2 * cus / std::max<uint64_t>(rest, 1), S / 32, cap}));
+            if (main_units == 0 && MB == 1) kc = std::max(kc, two_kc);
             while (kc > 1 && rest * kc * BM * kPcW > kPartialFloats) --kc;
             if (kc < 2) main_units = units;  // nothing to gain: one launch
         }

@@ -11,9 +11,11 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("t", [Q4_K, Q6_K])
-# 33 / 3 / 12 tiles of 128 rows; 4, 8, 9 and 17 super-blocks of K
-@pytest.mark.parametrize("rows,cols", [(4200, 1024), (300, 2048), (1500, 2304), (1472, 4352)])
-@pytest.mark.parametrize("n_vec", [33, 64])
+# 33 / 3 / 12 tiles of 128 rows (4, 8, 9 and 17 super-blocks of K), then half the chip's tiles and one more:
+# split up to there on every tile height, above it on 64-row tiles only
+@pytest.mark.parametrize("rows,cols,n_vec", [(4200, 1024, 33), (4200, 1024, 64), (300, 2048, 64), (1500, 2304, 33),
+                                             (1472, 4352, 64), (16384, 2048, 64), (16448, 2048, 40), (16384, 1024, 100),
+                                             (16448, 1024, 100)])
 def test_split_for_two_workgroups(hl, oracle, dev, t, rows, cols, n_vec):
     import torch
 
