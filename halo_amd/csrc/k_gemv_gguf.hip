@@ -26,9 +26,9 @@ using namespace dev;
 //     products of a 32-element slot that lane j takes (elements j, j + 8, j + 16, j + 24) need one
 //     16-byte read; two buffers, one barrier per chunk;
 //   - every weight is decoded once per launch and vector group and used for NV vectors.
-// With 8 or 16 vectors a lane takes two rows (when that still fills the chip), so each 16-byte read
-// of x feeds 16 instructions: with one row the LDS path (8 cycles per read and CU) and the four
-// SIMDs' 8 multiply-adds would be equally busy.
+// With 8 or 16 vectors a lane takes two rows, so each 16-byte read of x feeds 16 instructions: with
+// one row the LDS path (8 cycles per read and CU) and the four SIMDs' 8 multiply-adds would be
+// equally busy.
 //
 // Measured on MI355X against one thread per sum with byte loads and every weight decoded once per
 // vector: IQ4_NL 5120 x 17408 at 1 vector 646 -> 62 us, Q3_K 17408 x 5120 at 64 vectors 14470 ->
@@ -391,29 +391,40 @@ void launch_ref_nv(const RefArgs& a, uint32_t t0, uint32_t n, hipStream_t st) {
 
 template <uint32_t T>
 void launch_ref(const RefArgs& a, uint32_t n_vec, hipStream_t st) {
-    // groups of 16 vectors, then the smallest form that takes the rest in one launch
-    const uint32_t many = n_vec / 16 * 16, rest = n_vec - many;
-    // two rows per lane once that leaves about one wave per SIMD (1024 SIMDs x 16 rows)
-    const auto two = [&](uint32_t groups) { return (uint64_t)a.rows * groups >= 16 * 1024; };
-    if (many) {
-        if (two(many / 16)) launch_ref_nv<T, 16, 2>(a, 0, many, st);
-        else launch_ref_nv<T, 16, 1>(a, 0, many, st);
+    // Large groups decode least and small ones fill the chip soonest: a group's time hardly depends on
+    // its rows until there is about a wave per SIMD (1024). So: groups of 16 vectors with two rows per lane
+    // where those are 1024 waves; one of 8 for what is left of a large matrix; then groups of 4, or of 2
+    // while 4 would be fewer than 1024 waves. Measured on MI355X against groups of 16 and 8 everywhere, us:
+    // IQ4_NL 5120 x 17408 at 4 / 8 / 16 / 32 vectors 177 / 242 / 464 / 461 -> 110 / 184 / 211 / 383; Q3_K 1024 x
+    // 5120 45 / 55 / 130 / 131 -> 40 / 41 / 41 / 48; F16 6144 x 5120 40 / 78 / 137 / 143 -> 31 / 42 / 82 / 124.
+    uint32_t t = 0;  // vectors done
+    const uint32_t g16 = n_vec / 16 + (n_vec % 16 > 8 ? 1 : 0);
+    if ((uint64_t)a.rows * g16 >= 16 * 1024) {
+        t = std::min(n_vec, 16 * g16);
+        launch_ref_nv<T, 16, 2>(a, 0, t, st);
     }
-    if (rest > 8) {
-        if (two(1)) launch_ref_nv<T, 16, 2>(a, many, rest, st);
-        else launch_ref_nv<T, 16, 1>(a, many, rest, st);
-    } else if (rest > 4) {
-        if (two(1)) launch_ref_nv<T, 8, 2>(a, many, rest, st);
-        else launch_ref_nv<T, 8, 1>(a, many, rest, st);
-    } else if (rest > 2) {
-        launch_ref_nv<T, 4, 1>(a, many, rest, st);
-    } else if (rest == 2) {
-        launch_ref_nv<T, 2, 1>(a, many, rest, st);
-    } else if (rest == 1) {
+    if (n_vec - t > 4 && n_vec - t <= 8 && a.rows >= 32 * 1024) {
+        launch_ref_nv<T, 8, 2>(a, t, n_vec - t, st);
+        t = n_vec;
+    }
+    if (n_vec - t > 2) {
+        const uint32_t left = n_vec - t;
+        if ((uint64_t)a.rows * ((left + 1) / 4) >= 8 * 1024) {
+            const uint32_t n = std::min(left, (left + 1) / 4 * 4);  // the last group may be of 3
+            launch_ref_nv<T, 4, 1>(a, t, n, st);
+            t += n;
+        } else {
+            launch_ref_nv<T, 2, 1>(a, t, left / 2 * 2, st);
+            t += left / 2 * 2;
+        }
+    }
+    if (n_vec - t == 2) {
+        launch_ref_nv<T, 2, 1>(a, t, 2, st);
+    } else if (n_vec - t == 1) {
         if (a.rows <= kOneMaxRows)
-            hipLaunchKernelGGL((k_gemv_gguf_one<T>), dim3((a.rows - 1) / 8 + 1), dim3(64 * (kOneProducers + 1)), 0, st, a.w,
-                               a.w_stride, a.x + (uint64_t)many * a.x_stride, a.y + (uint64_t)many * a.y_stride, a.rows, a.cols);
-        else launch_ref_nv<T, 1, 1>(a, many, rest, st);
+            hipLaunchKernelGGL((k_gemv_gguf_one<T>), dim3((a.rows - 1) / 8 + 1), dim3(64 * (kOneProducers + 1)), 0, st, a.w, a.w_stride,
+                               a.x + (uint64_t)t * a.x_stride, a.y + (uint64_t)t * a.y_stride, a.rows, a.cols);
+        else launch_ref_nv<T, 1, 1>(a, t, 1, st);
     }
 }
 

@@ -22,7 +22,7 @@ def check(hl, oracle, dev, t, rows, cols, n_vec, pad=0, off=0, xp=0, yp=0, scale
 
 
 @pytest.mark.parametrize("t", GGUF_TYPES)
-@pytest.mark.parametrize("n_vec", [1, 2, 3, 5, 9, 17, 40])
+@pytest.mark.parametrize("n_vec", [1, 2, 3, 4, 5, 7, 9, 17, 40])
 def test_vector_groups(hl, oracle, dev, t, n_vec):
     # 1280 columns: a whole 1024-element chunk and a part of one; 9 rows: a wave's 8 and one more
     pad, off = (4, 4) if t == F32 else (3, 1)  # (F32 rows are 4-byte aligned)
@@ -30,10 +30,10 @@ def test_vector_groups(hl, oracle, dev, t, n_vec):
 
 
 @pytest.mark.parametrize("t", [Q3_K, Q6_K, IQ4_NL, Q8_0, F16, F32])
-@pytest.mark.parametrize("n_vec", [7, 16])
-def test_two_rows_per_lane(hl, oracle, dev, t, n_vec):
-    # 16385 rows: the two-row forms, one row past a whole workgroup of 64
-    check(hl, oracle, dev, t, 16385, BLOCK[t][0] if BLOCK[t][0] > 32 else 32, n_vec)
+@pytest.mark.parametrize("rows,n_vec", [(16385, 16), (16385, 21), (32769, 7)])
+def test_two_rows_per_lane(hl, oracle, dev, t, rows, n_vec):
+    # the two-row forms of 16 and 8 vectors, one row past a whole workgroup of 64
+    check(hl, oracle, dev, t, rows, BLOCK[t][0] if BLOCK[t][0] > 32 else 32, n_vec)
 
 
 @pytest.mark.parametrize("t", PLAIN_TYPES)
@@ -72,3 +72,10 @@ def test_one_vector_rounds(hl, oracle, dev, t, rows, cols):
     """One vector with the products made ahead (up to 6144 rows): fewer chunks than producers, an odd last
     round, more rounds than are loaded ahead, and the rows on either side of the rule."""
     check(hl, oracle, dev, t, rows, cols, 1)
+
+
+@pytest.mark.parametrize("t", [Q3_K, IQ4_NL, F16])
+@pytest.mark.parametrize("n_vec", [3, 4, 7, 11, 13, 14])
+def test_groups_of_four(hl, oracle, dev, t, n_vec):
+    """Enough rows for groups of four vectors (a last one of three, and what two and one are left)."""
+    check(hl, oracle, dev, t, 8200, 256, n_vec)
