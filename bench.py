@@ -544,7 +544,7 @@ def main() -> int:
         extra["q4k_17408x5120_repack_device"] = {"us": round(r["repack_us"], 2), "GB/s": round(r["repack_gbs"], 1),
                                                   "note": "reads + writes the 50 MB matrix once"}
         extra["q4k_17408x5120_upload_from_pinned_host"] = {"ms": round(r["upload_ms"], 3), "GB/s": round(r["upload_gbs"], 1),
-                                                           "note": "PCIe-inclusive, 64 MiB chunks through one staging buffer"}
+                                                           "note": "PCIe-inclusive, in chunks through a staging ring"}
         extra["q4k_17408x5120_upload_from_pageable_host"] = {"ms": round(r["pageable_ms"], 3),
                                                              "GB/s": round(r["pageable_gbs"], 1),
                                                              "note": "as from an mmap'd GGUF file"}
