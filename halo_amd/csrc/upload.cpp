@@ -205,6 +205,7 @@ int halo_mi_upload_tensors(const halo_mi_upload_tensor* tensors, uint32_t n, uin
         const uint64_t rb = halo_mi_row_bytes(tensors[i].type, tensors[i].cols);
         uint64_t rows = 0;
         for (uint32_t p = 0; p < tensors[i].n_parts; ++p) rows += tensors[i].parts[p].rows;
+        if (rows * rb == 0) continue;  // nothing to move (no rows, or rows of no columns)
         uint64_t chunk_rows = std::max<uint64_t>(chunk_bytes / rb / kSlabRows, 1) * kSlabRows;
         chunk_rows = std::min<uint64_t>(chunk_rows, (rows + kSlabRows - 1) / kSlabRows * kSlabRows);
         slot_bytes = std::max(slot_bytes, chunk_rows * rb);
@@ -227,6 +228,7 @@ int halo_mi_upload_tensors(const halo_mi_upload_tensor* tensors, uint32_t n, uin
         const uint64_t rb = halo_mi_row_bytes(tensors[i].type, tensors[i].cols);
         uint64_t rows = 0;
         for (uint32_t p = 0; p < tensors[i].n_parts; ++p) rows += tensors[i].parts[p].rows;
+        if (rows * rb == 0) continue;
         const uint64_t cr = std::max<uint64_t>(slot_bytes / rb / kSlabRows, 1) * kSlabRows;
         total_chunks += (rows + cr - 1) / cr;
     }
@@ -247,6 +249,7 @@ int halo_mi_upload_tensors(const halo_mi_upload_tensor* tensors, uint32_t n, uin
         const uint64_t rb = halo_mi_row_bytes(t.type, t.cols);
         uint64_t rows = 0;
         for (uint32_t p = 0; p < t.n_parts; ++p) rows += t.parts[p].rows;
+        if (rows * rb == 0) continue;
         const uint64_t chunk_rows = std::min<uint64_t>(std::max<uint64_t>(slot_bytes / rb / kSlabRows, 1) * kSlabRows,
                                                        (rows + kSlabRows - 1) / kSlabRows * kSlabRows);
         const SlabGeom g = slab_geom(t.type, t.cols);

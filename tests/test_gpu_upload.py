@@ -72,6 +72,23 @@ def test_upload_tensors_large_default_chunks(hl, dev):
     assert torch.equal(dst, ref)
 
 
+@pytest.mark.parametrize("empty", [(0, 512), (0, 0), (3, 0)])
+def test_upload_tensors_beside_empty_ones(hl, dev, empty):
+    """Tensors of no rows or no columns around a real one: the real one is uploaded, nothing else is written."""
+    import torch
+
+    t, rows, cols = Q6_K, 70, 512
+    say("upload_tensors beside empty", empty)
+    buf, _ = make_weights(t, rows, cols, seed=11)
+    w = buf[:rows * row_bytes(t, cols)]
+    dst = torch.full((hl.slab_bytes(t, rows, cols),), 0xCD, dtype=torch.uint8, device=dev)
+    other = torch.full((256,), 0xCD, dtype=torch.uint8, device=dev)
+    none = (Q4_K, empty[1], [(w, empty[0])], other)
+    hl.upload_tensors([none, (t, cols, [(w, rows)], dst), none])
+    assert np.array_equal(host(dst), hl.repack_slab_host(t, w, rows, cols))
+    assert torch.all(other == 0xCD)
+
+
 def test_upload_tensors_rejects(hl, dev):
     import torch
 

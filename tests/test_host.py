@@ -219,3 +219,24 @@ def test_single_hip_runtime_in_process(hl):
     import torch  # noqa: F401
 
     assert len(hl._lib.hip_runtimes()) == 1
+
+
+@pytest.mark.parametrize("rows,cols", [(0, 256), (0, 0), (3, 0)])
+def test_upload_of_nothing(hl, rows, cols):
+    """A tensor of no rows or no columns uploads as nothing, alone or beside others of its kind: no GPU call
+    is made. In a process of its own, since a fault here is a signal."""
+    import subprocess
+    import sys
+
+    code = f"""
+import ctypes
+import halo_amd as hl
+mem = ctypes.create_string_buffer(64)
+at = (ctypes.addressof(mem) + 15) // 16 * 16
+t = int(hl.DType.Q4_K)
+hl.upload_slab(t, at, {rows}, {cols}, at, stream=0)
+hl.upload_tensors([(t, {cols}, [(at, {rows})], at), (t, 0, [(at, 0)], at), (t, 256, [(at, 0), (at, 0)], at)], stream=0)
+print("done")
+"""
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and r.stdout.strip() == "done", r
