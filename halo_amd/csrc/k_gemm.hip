@@ -594,19 +594,22 @@ __device__ __forceinline__ void gemm_pc_body(const GemmPcArgs& a, uint32_t bid, 
             }
         }
         if (split) {
-            // fp32 partial tile [BM][128] of this chunk; the reduce reads only the rows of x, so a
-            // tile's padding rows are not written (MI355X, Q6_K 5120 x 17408 at 140 / 200 / 270 rows of x:
-            // 58.2 / 61.2 / 98.0 -> 55.5 / 59.0 / 94.8 us; K = 5120 within the noise)
+            // fp32 partial tile [BM][128] of this chunk. The reduce reads only the rows of x, so in chunks of 5
+            // super-blocks and more the 32-row blocks past them are not written (MI355X, 17408 columns, 5120 rows
+            // of W at 129 / 160 / 200 / 300 rows of x: 5 / 5 / 3 / 3% less time; in chunks of one to 4, as 5120 rows of
+            // 2048 and 5120 columns have, 2-3% more at 129-200 rows. A test per row cost 1-5% in both).
+            const uint32_t written = n >= 40 ? a.n_vec - m0 : BM;
             float* P = a.partials + ((uint64_t)st * a.kchunks + chunk) * BM * kPcW;
 #pragma unroll
-            for (int i = 0; i < MBW; ++i)
+            for (int i = 0; i < MBW; ++i) {
+                if ((wm * MBW + i) * 32 >= written) break;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const uint32_t ml = (wm * MBW + i) * 32 + mfma32_row(r, lane);
-                    if (m0 + ml >= a.n_vec) continue;
 #pragma unroll
                     for (int j = 0; j < NBW; ++j) P[ml * kPcW + wrow[j] + lr] = acc[i][j][r];
                 }
+            }
             return;
         }
         // epilogue: columns of this lane, rows m per accumulator element

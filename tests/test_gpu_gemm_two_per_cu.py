@@ -4,8 +4,8 @@ GEMM's accumulation bound."""
 import numpy as np
 import pytest
 
-from helpers import Q4_K, Q6_K, gemm_emulated, make_weights
-from test_gpu_parity import host, say, to_dev
+from helpers import Q4_K, Q6_K, gemm_emulated, make_weights, synth_matrix
+from test_gpu_parity import SENTINEL, host, say, to_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -32,3 +32,23 @@ def test_split_for_two_workgroups(hl, oracle, dev, t, rows, cols, n_vec):
     size = rows * cols // 256 * (144 if t == Q4_K else 210)
     ref, tol = gemm_emulated(oracle, t, buf[:size], rows, cols, x)
     assert np.all(np.abs(got - ref) <= tol)
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q6_K])
+# chunks of 4 and of 5 super-blocks on 128- and 256-row tiles, whose 32-row blocks past x are written below 5 only
+@pytest.mark.parametrize("rows,cols,n_vec", [(4096, 8192, 65), (4096, 10240, 65), (4096, 10240, 129), (4096, 8192, 225)])
+def test_partials_of_part_of_a_tile(hl, oracle, dev, t, rows, cols, n_vec):
+    import torch
+
+    say("partials", t, rows, cols, n_vec)
+    w = synth_matrix(hl, t, rows, cols, seed=cols + n_vec)
+    x = np.random.default_rng(n_vec).normal(0, 1, (n_vec, cols)).astype(np.float32)
+    slab = torch.empty(hl.slab_bytes(t, rows, cols), dtype=torch.uint8, device=dev)
+    hl.repack_slab(t, to_dev(w, dev), rows, cols, slab)
+    y = torch.full((n_vec, rows + 3), SENTINEL, dtype=torch.float32, device=dev)
+    hl.gemv(t, slab, to_dev(x, dev), y, rows, cols, n_vec, y_stride=rows + 3, variant=3)
+    got = host(y)
+    assert np.all(got[:, rows:] == SENTINEL)
+    pick = np.r_[0:64, rows - 192:rows]
+    ref, tol = gemm_emulated(oracle, t, w.reshape(rows, -1)[pick].reshape(-1), pick.size, cols, x)
+    assert np.all(np.abs(got[:, pick] - ref) <= tol)
