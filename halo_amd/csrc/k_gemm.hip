@@ -1418,6 +1418,37 @@ int launch_gemm_sm(uint32_t type, const GemmArgs& a, Workspace* ws, uint32_t uni
     return hip_status(hipGetLastError(), "gemm_sm launch");
 }
 
+// K chunks per tile where k_gemm_pc's tiles are less than one round of the chip (1: whole tiles).
+// One workgroup per CU: as many chunks as the CUs hold below half a round; at half a round 2, if those have
+// at least 8 super-blocks (MI355X, 128 tiles of 128 and of 256 rows, us whole and in 2: 1024 columns 16 / 25 and 24 /
+// 35, 2048 24 / 29 and 33 / 41, 3072 32 / 34 and 43 / 48; from 4096 columns on 2 are faster: gate/up of 5120
+// 50 / 41 and 64 / 54).
+// Two per CU, on 64-row tiles (128- and 256-row ones measured slower): one's stage barriers hide behind the
+// other's work, but more partials are written and added. Taken with chunks of at least 4 super-blocks where
+// the busiest CU's super-blocks fall by a tenth, or with at least 5 (10 where the tiles would be whole, with no
+// partials at all) where they rise by 6% at most. Measured, time with two per CU over time with one, M = 64, Q4_K
+// and Q6_K, the worst of plain and pair (in brackets: not taken):
+//   tiles              40     56     64     80     96    112    127    128    160    192    224    255
+//   17408 columns    0.93   0.87   0.94   0.87   0.75   0.84   0.85   0.51   0.64   0.83   0.84   0.85
+//   8192           (1.05) (1.02) (1.04) (0.97)   0.86   0.92   0.92   0.61   0.70   0.89   0.89   0.90
+//   5120                - (1.19) (1.19) (1.05)   0.95   0.98   0.98   0.74   0.82   0.96   0.97   0.98
+//   4096                -      -      - (1.07) (1.00) (1.01) (1.03)   0.81   0.90 (1.00) (1.02) (1.03)
+//   3072                -      -      -      - (1.11) (1.11) (1.11)   0.92   0.97 (1.07) (1.09) (1.11)
+//   2048                -      -      -      -      -      -      -   0.96 (1.14) (1.18) (1.23) (1.26)
+uint32_t all_split_chunks(uint64_t tiles, uint32_t blocks, uint32_t cus, bool two_fit) {
+    if (tiles == 0) return 1;
+    uint32_t one = 1;
+    if (2 * tiles < cus) one = (uint32_t)std::min<uint64_t>({cus / tiles, blocks, 16});
+    else if (2 * tiles == cus && !two_fit && blocks >= 16) one = 2;
+    if (!two_fit) return one;
+    const uint32_t two = (uint32_t)std::min<uint64_t>({2 * cus / tiles, blocks / 4, 16});
+    if (two <= one) return one;
+    // super-blocks of the busiest CU
+    auto share = [&](uint32_t k) { return (uint64_t)((blocks + k - 1) / k) * ((tiles * k + cus - 1) / cus); };
+    const uint64_t s1 = share(one), s2 = share(two);
+    return 11 * s2 <= 10 * s1 || (50 * s2 <= 53 * s1 && blocks / two >= (one > 1 ? 5u : 10u)) ? two : one;
+}
+
 }  // namespace
 
 // x -> bf16 staging (in chunks of rows that fit the workspace), then the GEMM: k_gemm_sm for at
@@ -1473,34 +1504,25 @@ int launch_gemm_pc(uint32_t type, const GemmArgs& a, hipStream_t st) {
         const uint32_t m_tiles = (mc + BM - 1) / BM;
         if (int rc = stage_x(a, m_start, mc, m_tiles * BM, ws, st)) return rc;
         float* y = a.y + m_start * a.y_stride;
-        // whole rounds of tiles, then the rest split over K; a matrix whose tiles fill at most half
-        // the chip is split over K altogether, and on 64-row tiles so is one of less than a whole round
-        // that has two chunks or more to fill two workgroups per CU with (MI355X, Q4_K gate/up pairs
-        // of 5120 columns, M = 64, us whole and split: 128 units 46 -> 32 with 4 chunks, 160 47 -> 38
-        // with 3, 224 50 -> 45 and 255 49 -> 47 with 2; M = 128 / 256: 128 units 50 / 64 -> 41 / 54,
-        // 160 and more no faster; 256 units at M = 64 44 -> 46)
+        // whole rounds of tiles, then the rest split over K; with less than a round every tile is whole or
+        // every one is split (all_split_chunks)
         const uint64_t tiles = (uint64_t)units * m_tiles;
         uint32_t main_units = units, kc = 1;
-        const uint32_t two_kc = (uint32_t)std::min<uint64_t>({2 * cus / std::max<uint64_t>(tiles, 1), S / 32, 16});
-        if (S % 8 == 0 && ((tiles > cus && tiles % cus != 0) || 2 * tiles <= cus || (MB == 1 && tiles < cus && two_kc >= 2))) {
-            main_units = tiles > cus ? (uint32_t)(tiles / cus * cus / m_tiles) : 0u;
+        if (S % 8 == 0 && tiles < cus) {
+            kc = all_split_chunks(tiles, S / 8, cus, MB == 1);
+            main_units = 0;
+        } else if (S % 8 == 0 && tiles % cus != 0) {
+            main_units = (uint32_t)(tiles / cus * cus / m_tiles);
             const uint64_t rest = (uint64_t)(units - main_units) * m_tiles;
             // Tiles left over beside a whole round: 64-row tiles run two workgroups per CU, so
             // their chunks run beside the whole tiles and 2 chunks suffice (the fewer partials,
             // the shorter the reduce); larger tiles hold a CU alone, so their chunks run after
             // the round and 8 keep that tail short (measured on MI355X, gate/up 17408 x 5120:
             // M = 64 57.3 -> 49.0 us, M = 128 70.4 -> 68.4, M = 256 105.2 -> 102.5, against 16)
-            const uint32_t cap = main_units == 0 ? 16u : (MB == 1 ? 2u : 8u);
-            kc = (uint32_t)std::min<uint64_t>({cus / std::max<uint64_t>(rest, 1), S / 8, cap});
-            // Every tile split, 64-row tiles: two workgroups fit a CU, and with both there one's stage
-            // barriers hide behind the other's work, as long as a chunk has at least 4 super-blocks
-            // (MI355X, M = 64, us at one and two workgroups per CU: Q5_K 12288 x 5120 34.8 -> 31.5 with 5
-            // chunks, Q6_K 5120 x 17408 41.5 -> 38.2 with 12; with 2 super-blocks per chunk Q5_K 5120 x
-            // 6144 23.3 -> 25.4, Q4_K 6144 x 5120 21.5 -> 24.1). 128- and 256-row tiles measured slower.
-            if (main_units == 0 && MB == 1) kc = std::max(kc, two_kc);
-            while (kc > 1 && rest * kc * BM * kPcW > kPartialFloats) --kc;
-            if (kc < 2) main_units = units;  // nothing to gain: one launch
+            kc = (uint32_t)std::min<uint64_t>({cus / std::max<uint64_t>(rest, 1), S / 8, MB == 1 ? 2u : 8u});
         }
+        while (kc > 1 && (uint64_t)(units - main_units) * m_tiles * kc * BM * kPcW > kPartialFloats) --kc;
+        if (kc < 2) main_units = units;  // nothing to gain: one launch
         // one launch: the whole tiles, then the split tiles' chunks (dispatched as CUs free up)
         GemmPcArgs p{a.w0, a.w1, ws->xb, y, a.y_stride, a.rows, a.cols, mc, main_units, m_tiles, 0u,
                      units - main_units, kc, ws->partials};
@@ -1553,10 +1575,11 @@ bool gemm_group_types(uint32_t ta, uint32_t tb, const GemmGroupArgs& g, dim3 gri
 }
 
 // One launch over the segments of weight types ta and tb on the staged rows (mc of them, m_tiles
-// M tiles of 64 MB rows): whole tiles when they fill half the GPU or more (as k_gemm_pc's
-// choice), else every tile split over the same K chunks into the workspace's partials, then one
-// reduce over all of them. (Config 5's q|k|v at M = 512 is 128 whole tiles; two K chunks each
-// plus the reduce measured 533.0 against 531.3 us for the whole layer, same box.)
+// M tiles of 64 MB rows): whole tiles when they fill half the GPU or more, else every tile split over the
+// same K chunks, for one workgroup per CU, into the workspace's partials, then one reduce over all of them.
+// (Config 5's q|k|v at M = 512 is 128 whole tiles; two K chunks each plus the reduce measured 533.0 against
+// 531.3 us for the whole layer, same box. At M = 64 it is 64 tiles of 20 super-blocks, which all_split_chunks
+// gives the same 4 chunks.)
 template <int MB>
 int gemm_group_launch(const GroupSeg* segs, uint32_t n, uint32_t ta, uint32_t tb, uint32_t cols, uint32_t mc, uint32_t m_tiles,
                       uint64_t m_start, Workspace* ws, hipStream_t st) {
