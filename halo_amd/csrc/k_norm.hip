@@ -3,9 +3,10 @@
 //   mean = dot(x, x) / cols   (cpu::detail::dot, backends/cpu/kernel_common.h:16-27)
 //   inv  = 1 / sqrt(mean + eps)
 //   out  = (x * inv) * w
-// Both kernels compute the sum of squares in the CPU's order, so the results are bitwise the
+// Every kernel computes the sum of squares in the CPU's order, so the results are bitwise the
 // CPU's: k_rms_norm_rows writes the normalized rows (the reference-order GEMV's input, and the
-// RMS_NORM op itself); k_rms_inv_rows writes only inv per row, for the GEMM's x staging.
+// RMS_NORM op itself); k_norm_to_frag writes them in bf16 as the GEMM's staged x, and k_rms_inv_rows
+// only inv per row, for rows too wide for that.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -20,6 +21,7 @@ namespace halo_mi {
 namespace {
 
 constexpr uint32_t kNormBlock = 512;
+constexpr uint32_t kNormManyBlock = 256;  // for more rows than fit at once (launch_rms_norm)
 constexpr uint32_t kNormChunk = 8192;  // floats of a row staged in LDS at a time
 constexpr uint32_t kChainStride = dev::norm_chain_stride(kNormChunk);  // LDS floats per chain row (padded)
 constexpr uint32_t kNormLds = dev::norm_lds_floats(kNormChunk);        // the chain rows, then the result
@@ -28,10 +30,10 @@ constexpr uint32_t kNormLds = dev::norm_lds_floats(kNormChunk);        // the ch
 // (norm_device.h): each chunk's squares are staged in LDS transposed (every load of the chunk is
 // issued before the first is used: one memory round trip per chunk), lanes 0..7 of wave 0 carry
 // the 8 chain sums across the chunks, then wave 0 combines them and thread 0 finishes. PT: loads
-// per thread and chunk, PT * kNormBlock >= min(cols, kNormChunk). v: the last chunk's elements,
-// v[i] at tid + i * kNormBlock (the whole row when it is one chunk); `meanwhile` runs while the
+// per thread and chunk, PT * BLOCK >= min(cols, kNormChunk). v: the last chunk's elements,
+// v[i] at tid + i * BLOCK (the whole row when it is one chunk); `meanwhile` runs while the
 // chains do, after the last chunk's loads.
-template <uint32_t PT, typename F>
+template <uint32_t BLOCK, uint32_t PT, typename F>
 __device__ __forceinline__ float row_rms_inv(const float* __restrict__ x, uint32_t cols, float eps, float* lds, float (&v)[PT],
                                              F meanwhile) {
 #pragma clang fp contract(off)
@@ -41,11 +43,11 @@ __device__ __forceinline__ float row_rms_inv(const float* __restrict__ x, uint32
     for (uint32_t c0 = 0; c0 < cols; c0 += kNormChunk) {
         const uint32_t here = min(kNormChunk, cols - c0), n = min(here, full - min(c0, full));  // n: a multiple of 8
 #pragma unroll
-        for (uint32_t i = 0; i < PT; ++i) v[i] = x[c0 + min(tid + i * kNormBlock, here - 1)];  // past the end: not used
+        for (uint32_t i = 0; i < PT; ++i) v[i] = x[c0 + min(tid + i * BLOCK, here - 1)];  // past the end: not used
         if (c0 + here == cols) meanwhile();
 #pragma unroll
         for (uint32_t i = 0; i < PT; ++i) {
-            const uint32_t e = tid + i * kNormBlock;
+            const uint32_t e = tid + i * BLOCK;
             if (e < n) lds[(e % 8) * kChainStride + e / 8] = v[i] * v[i];
         }
         __syncthreads();
@@ -60,13 +62,13 @@ __device__ __forceinline__ float row_rms_inv(const float* __restrict__ x, uint32
     return lds[8 * kChainStride];
 }
 
-// grid rows, block kNormBlock. out may be x (each element is read before it is written, by
-// the same thread, after the whole row has been summed). A row of one chunk stays in registers,
+// grid rows, block BLOCK. out may be x (each element is read before it is written, by
+// the same thread, after the whole row has been summed). KEEP: a row of one chunk stays in registers,
 // and the norm weights are loaded before the chains: what remains is the row's one round trip to
 // memory and the chains (3 rows of 5120: 7.3 -> 5.6 us in the kernel trace, against 256 threads that
-// read the row again for the output; 512 rows 11.0 -> 9.0).
-template <uint32_t PT>
-__global__ __launch_bounds__(kNormBlock) void k_rms_norm_rows(const float* x, uint64_t x_stride,
+// read the row again for the output; 512 rows 11.0 -> 9.0). Else the row is read again for the output.
+template <uint32_t BLOCK, uint32_t PT, bool KEEP>
+__global__ __launch_bounds__(BLOCK) void k_rms_norm_rows(const float* x, uint64_t x_stride,
                                                               const float* __restrict__ w, float* out,
                                                               uint64_t out_stride, uint32_t cols, float eps) {
 #pragma clang fp contract(off)
@@ -74,23 +76,27 @@ __global__ __launch_bounds__(kNormBlock) void k_rms_norm_rows(const float* x, ui
     const float* xr = x + (uint64_t)blockIdx.x * x_stride;
     float* o = out + (uint64_t)blockIdx.x * out_stride;
     const uint32_t tid = threadIdx.x;
-    const bool one = cols <= kNormChunk;
+    const bool one = KEEP && cols <= kNormChunk;
     float v[PT], wv[PT];
-    auto load_w = [&](uint32_t c0, uint32_t n) __attribute__((always_inline)) {
+    const float inv = row_rms_inv<BLOCK, PT>(xr, cols, eps, lds, v, [&]() __attribute__((always_inline)) {
+        if (one) {
 #pragma unroll
-        for (uint32_t i = 0; i < PT; ++i) wv[i] = w[c0 + min(tid + i * kNormBlock, n - 1)];
-    };
-    const float inv = row_rms_inv<PT>(xr, cols, eps, lds, v, [&]() __attribute__((always_inline)) { if (one) load_w(0, cols); });
+            for (uint32_t i = 0; i < PT; ++i) wv[i] = w[min(tid + i * BLOCK, cols - 1)];
+        }
+    });
     for (uint32_t c0 = 0; c0 < cols; c0 += kNormChunk) {
         const uint32_t n = min(kNormChunk, cols - c0);
         if (!one) {  // every load of a chunk before the first store: one memory round trip per chunk
-            load_w(c0, n);
 #pragma unroll
-            for (uint32_t i = 0; i < PT; ++i) v[i] = xr[c0 + min(tid + i * kNormBlock, n - 1)];
+            for (uint32_t i = 0; i < PT; ++i) {
+                const uint32_t e = c0 + min(tid + i * BLOCK, n - 1);
+                v[i] = xr[e];
+                wv[i] = w[e];
+            }
         }
 #pragma unroll
         for (uint32_t i = 0; i < PT; ++i) {
-            const uint32_t e = tid + i * kNormBlock;
+            const uint32_t e = tid + i * BLOCK;
             if (e < n) {
                 const float t = v[i] * inv;
                 o[c0 + e] = t * wv[i];
@@ -104,7 +110,7 @@ __global__ __launch_bounds__(kNormBlock) void k_rms_inv_rows(const float* __rest
                                                              uint32_t cols, float eps, float* __restrict__ inv) {
     __shared__ float lds[kNormLds];
     float v[PT];
-    const float s = row_rms_inv<PT>(x + (uint64_t)blockIdx.x * x_stride, cols, eps, lds, v, []() {});
+    const float s = row_rms_inv<kNormBlock, PT>(x + (uint64_t)blockIdx.x * x_stride, cols, eps, lds, v, []() {});
     if (threadIdx.x == 0) inv[blockIdx.x] = s;
 }
 
@@ -206,9 +212,18 @@ void with_loads(uint32_t cols, F f) {
 int launch_rms_norm(const float* x, uint64_t x_stride, const float* w, float* out, uint64_t out_stride, uint32_t rows,
                     uint32_t cols, float eps, hipStream_t st) {
     if (rows == 0 || cols == 0) return HALO_MI_OK;
-    with_loads(cols, [&](auto pt) {
-        hipLaunchKernelGGL(k_rms_norm_rows<pt()>, dim3(rows), dim3(kNormBlock), 0, st, x, x_stride, w, out, out_stride, cols, eps);
-    });
+    // A kept row costs registers: with 16 loads per thread (above 6144 columns) a CU holds one
+    // workgroup, with 6 to 12 two, where the form that reads the row again holds four. So rows that would
+    // wait for a second round of those take that form (MI355X, kept over read again: 8192 columns 0.84 at 256 rows,
+    // 1.26 at 257, 1.24 at 512, 1.54 at 520, 1.70 at 3000; 5120 columns 0.82 at 512, 1.07 at 520, 1.11 at 3000; 4096
+    // 0.77 at 512, 1.01 at 520, 1.08 at 700, 1.11 at 3000; 3072 1.00 at 1024, 1.07 at 3000; 2048 0.65 at 512, 0.63 at 3000).
+    const bool many = cols > 6144 ? rows > 256 : cols > 3072 ? rows > 512 : cols > 2048 && rows > 1024;
+    auto launch = [&](auto kernel, uint32_t block) {
+        hipLaunchKernelGGL(kernel, dim3(rows), dim3(block), 0, st, x, x_stride, w, out, out_stride, cols, eps);
+    };
+    if (many && cols > 6144) launch(k_rms_norm_rows<kNormManyBlock, 32, false>, kNormManyBlock);
+    else if (many) launch(k_rms_norm_rows<kNormManyBlock, 24, false>, kNormManyBlock);
+    else with_loads(cols, [&](auto pt) { launch(k_rms_norm_rows<kNormBlock, pt(), true>, kNormBlock); });
     return hip_status(hipGetLastError(), "rms_norm launch");
 }
 

@@ -534,3 +534,21 @@ def test_gemv_group_rejects(hl, dev):
     with pytest.raises(hl.HaloError) as e:
         hl.gemv_group([(Q4_K, w, 64, y)] * 5, x, cols, 1)
     assert e.value.code == hl.ErrorCode.Unsupported
+
+
+# rows around the ones that stay in registers (256, 512, 1024 by width) and the widths where that changes
+@pytest.mark.parametrize("rows,cols", [(256, 8192), (257, 6145), (300, 8193), (257, 17408), (512, 6144), (513, 6144),
+                                       (513, 4097), (512, 4096), (513, 3073), (1024, 3072), (1025, 2049), (1030, 2048)])
+def test_rms_norm_many_rows_bitwise(hl, oracle, dev, rows, cols):
+    import torch
+
+    say("rms_norm many", rows, cols)
+    x, w = norm_inputs(cols, rows, rows + cols)
+    ref = oracle.rms_norm(x, w, EPS)
+    xd, wd = to_dev(x, dev), to_dev(w, dev)
+    out = torch.full((rows, cols + 1), SENTINEL, dtype=torch.float32, device=dev)
+    hl.rms_norm(xd, wd, out, rows, cols, eps=EPS, out_stride=cols + 1)
+    o = host(out)
+    assert isclose_bits(o[:, :cols], ref) and np.all(o[:, cols:] == SENTINEL)
+    hl.rms_norm(xd, wd, xd, rows, cols, eps=EPS)  # in place
+    assert isclose_bits(host(xd), ref)
