@@ -222,11 +222,13 @@ template <uint32_t T>
 bool norm_in_kernel_t(uint32_t slabs, uint32_t cols, uint32_t mats, bool have_ws) {
     const EvenSplit ev = pick_even<T>(slabs, cols / kSlot, mats, have_ws);
     const GemvSplit sp = pick_split<T>(slabs, cols / kSlot, mats, have_ws);
-    // Without split K nothing is published, and every workgroup would run the chains: with more
-    // workgroups than CUs that is paid once per round of them. The RMS_NORM kernel first then costs
-    // one launch (Q6_K 248320 x 5120 with its logits, MI355X: 247.6 -> 195.1 us). Few workgroups, or a call with
-    // no workspace to normalize into, keep the norm inside.
-    if (!ev.W && sp.ks * mats == 1 && slabs > 256 && have_ws) return false;
+    // Without split K nothing is published, and every workgroup runs the chains: with more workgroups
+    // than CUs that is paid once per round of them. The RMS_NORM kernel first costs one launch instead, which
+    // pays for long rows (MI355X, the norm before the GEMV over inside it, means of the types: 69632 rows of
+    // 512 / 768 / 1024 / 2048 / 5120 columns 1.13 / 1.06 / 1.04 / 0.89 / 0.87; 151936 rows 1.02 / 0.96 / 0.96 / 0.83 / 0.89; 256
+    // columns 1.08-1.23 from 16448 to 248320 rows; Q6_K 248320 x 5120 with its logits 247.6 -> 195.1 us). Few
+    // workgroups, or a call with no workspace to normalize into, keep the norm inside.
+    if (!ev.W && sp.ks * mats == 1 && slabs > 256 && cols > 1024 && have_ws) return false;
     const uint32_t nw = ev.W ? ev.nu : sp.nw;
     const size_t lds = ev.W ? even_lds_bytes<1>(ev.nu, nw) : mx_lds_bytes<1>(nw);
     const uint32_t full = cols - cols % 8u;

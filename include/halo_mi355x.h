@@ -160,7 +160,7 @@ enum {
  *        - SLAB GEMV (2 and the GEMV legs of the auto variants), one vector: inside the MFMA
  *          GEMV's launch, one dispatch: every workgroup computes 1 / rms in cpu::rms_norm's
  *          order and normalizes its own x elements as cpu::rms_norm rounds them (cols <= 8192;
- *          matrices of up to 256 slabs, or whose launch splits K over workgroups);
+ *          matrices of up to 256 slabs or 1024 columns, or whose launch splits K over workgroups);
  *        - otherwise (more vectors, wider rows, more slabs than that with K unsplit, variant 6): x
  *          is normalized into the stream's workspace by the RMS_NORM kernel, then the GEMV runs on it.
  *      So y is bitwise halo_mi_rms_norm then the same variant without the norm, at any n_vec

@@ -156,8 +156,8 @@ def test_gemv_norm_reference_variant_bitwise(hl, oracle, dev, t):
 
 
 # One vector with cols <= 8192 takes the norm inside the GEMV kernel (one dispatch: the norm wave
-# of the first workgroup publishes 1 / rms); more vectors, and the 17408-column row, the RMS_NORM
-# kernel then the GEMV. (17408, 5120, 1) is the headline shape (1088 workgroups of 5 + 1 waves);
+# of the first workgroup publishes 1 / rms); more vectors, the 17408-column row, and more than 256 slabs
+# of over 1024 columns with K unsplit (test_gemv_norm_unsplit_k), the RMS_NORM kernel then the GEMV. (17408, 5120, 1) is the headline shape (1088 workgroups of 5 + 1 waves);
 # 65600 rows: more than 1024 slabs (two groups per wave).
 NORM_CASES = [(130, 1024, 1), (130, 1024, 4), (576, 5120, 1), (576, 5120, 3), (640, 17408, 1), (70, 512, 6),
               (65600, 512, 1), (65600, 512, 4), (17408, 5120, 1), (64, 256, 1)]  # (64, 256, 1): one workgroup
@@ -552,3 +552,45 @@ def test_rms_norm_many_rows_bitwise(hl, oracle, dev, rows, cols):
     assert isclose_bits(o[:, :cols], ref) and np.all(o[:, cols:] == SENTINEL)
     hl.rms_norm(xd, wd, xd, rows, cols, eps=EPS)  # in place
     assert isclose_bits(host(xd), ref)
+
+
+@pytest.mark.parametrize("t", (Q4_K, Q6_K, Q8_0))
+@pytest.mark.parametrize("rows,cols", [(16400, 256), (69633, 1024), (69633, 1280)])
+def test_gemv_norm_unsplit_k(hl, oracle, dev, t, rows, cols):
+    """More than 256 slabs with K unsplit: up to 1024 columns the norm stays in the GEMV, above it runs first. Both are
+    bitwise RMS_NORM then the GEMV, plain, in the LM head, without allocation, and captured on a stream that has
+    no workspace (where the norm stays in the GEMV)."""
+    import torch
+
+    say("gemv norm unsplit", NAMES[t], rows, cols)
+    raw = np.tile(make_weights(t, 64, cols, seed=t)[0][:64 * row_bytes(t, cols)], (rows + 63) // 64)[:rows * row_bytes(t, cols)]
+    slab = slab_of(hl, dev, t, raw, rows, cols)
+    x, w = norm_inputs(cols, 1, cols)
+    xd, wd = to_dev(x, dev), to_dev(w, dev)
+    xn = to_dev(oracle.rms_norm(x, w, EPS), dev)
+    want = torch.full((1, rows), SENTINEL, dtype=torch.float32, device=dev)
+    hl.gemv(t, slab, xn, want, rows, cols, 1, variant=hl.Variant.SLAB_GEMV)
+    want = host(want)
+
+    def fresh():
+        return torch.full((1, rows), SENTINEL, dtype=torch.float32, device=dev)
+
+    y = fresh()
+    hl.gemv(t, slab, xd, y, rows, cols, 1, norm_w=wd, norm_eps=EPS)
+    assert isclose_bits(host(y), want)
+    y = fresh()
+    hl.gemv_noalloc(t, slab, xd, y, rows, cols, 1, norm_w=wd, norm_eps=EPS)
+    assert isclose_bits(host(y), want)
+    y, res = fresh(), torch.zeros((1, 3), dtype=torch.int32, device=dev)
+    hl.lm_head(t, slab, xd, res, rows, cols, 1, logits=y, norm_w=wd, norm_eps=EPS)
+    assert isclose_bits(host(y), want) and int(host(res)[0, 0]) == int(np.argmax(want[0]))
+    y, st = fresh(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=st):
+        hl.gemv(t, slab, xd, y, rows, cols, 1, norm_w=wd, norm_eps=EPS)
+    for _ in range(3):
+        y.fill_(SENTINEL)
+        g.replay()
+        torch.cuda.synchronize()
+        assert isclose_bits(host(y), want)
