@@ -33,31 +33,35 @@ __global__ __launch_bounds__(64) void k_argmax_parts(const float* __restrict__ l
     if (lane == 0) parts[(uint64_t)v * gridDim.x + p] = ArgPart{bv, bi, any_nan, 0u};
 }
 
-// grid n_vec, block kFinishBlock. A poisoned vector (any NaN logit) reports {kNoIndex, quiet NaN, 1}
+// grid n_vec, block BLOCK. A poisoned vector (any NaN logit) reports {kNoIndex, quiet NaN, 1}
 // (cpu_backend.cpp:745-747); one with no ranked row {kNoIndex, 0, 0} (TopKEntry's default,
 // include/halo/backends/cpu/ops.h:351-355). ids: the winning index, 0 for either of those
 // (cpu_backend.cpp:756-760); ids_scatter[ids_slots[v]] likewise, a slot past the end dropped.
 // Bound by its launch and one round trip to the parts: kFinishLoads of them are in flight per thread, so
 // a 248320-row head's 3880 parts take one round, and the ranking runs in registers (MI355X, that head
 // with one vector, norm and logits: 194.5 -> 190.6 us; ARGMAX alone over 248320 logits 9.6 -> 6.1; against 256
-// threads with one load at a time and a tree in LDS).
-constexpr uint32_t kFinishBlock = 1024, kFinishLoads = 4, kFinishWaves = kFinishBlock / 64;
-__global__ __launch_bounds__(kFinishBlock) void k_argmax_finish(const ArgPart* __restrict__ parts, uint32_t n_parts,
-                                                                uint32_t* __restrict__ result, int32_t* ids,
-                                                                const uint32_t* ids_slots, int32_t* ids_scatter,
-                                                                uint64_t scatter_len) {
-    __shared__ float sv[kFinishWaves];
-    __shared__ uint32_t si[kFinishWaves], sn[kFinishWaves];
+// threads with one load at a time and a tree in LDS). Up to 256 parts 256 threads hold them all: with many
+// vectors the idle waves of the larger block cost more than its loads save (512 vectors of 64 / 1000
+// logits 5.5 / 7.2 us with 256 threads, 6.0 / 7.8 with 1024).
+constexpr uint32_t kFinishBlock = 1024, kFinishSmallBlock = 256, kFinishLoads = 4;
+template <uint32_t BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_argmax_finish(const ArgPart* __restrict__ parts, uint32_t n_parts,
+                                                         uint32_t* __restrict__ result, int32_t* ids,
+                                                         const uint32_t* ids_slots, int32_t* ids_scatter,
+                                                         uint64_t scatter_len) {
+    constexpr uint32_t kWaves = BLOCK / 64, LOADS = BLOCK == kFinishSmallBlock ? 1 : kFinishLoads;
+    __shared__ float sv[kWaves];
+    __shared__ uint32_t si[kWaves], sn[kWaves];
     const uint32_t v = blockIdx.x, tid = threadIdx.x, lane = tid & 63u;
     const ArgPart* mine = parts + (uint64_t)v * n_parts;
     float bv = 0.0f;
     uint32_t bi = kNoIndex, nan = 0;
-    for (uint32_t i = tid; i < n_parts; i += kFinishBlock * kFinishLoads) {
-        ArgPart q[kFinishLoads];
+    for (uint32_t i = tid; i < n_parts; i += BLOCK * LOADS) {
+        ArgPart q[LOADS];
 #pragma unroll
-        for (uint32_t k = 0; k < kFinishLoads; ++k) q[k] = mine[min(i + k * kFinishBlock, n_parts - 1)];  // (a part twice ranks once)
+        for (uint32_t k = 0; k < LOADS; ++k) q[k] = mine[min(i + k * BLOCK, n_parts - 1)];  // (a part twice ranks once)
 #pragma unroll
-        for (uint32_t k = 0; k < kFinishLoads; ++k) {
+        for (uint32_t k = 0; k < LOADS; ++k) {
             nan |= q[k].nan;
             if (ranks_before(q[k].value, q[k].index, bv, bi)) {
                 bv = q[k].value;
@@ -75,7 +79,7 @@ __global__ __launch_bounds__(kFinishBlock) void k_argmax_finish(const ArgPart* _
     }
     __syncthreads();
     if (tid >= 64) return;
-    const bool held = lane < kFinishWaves;
+    const bool held = lane < kWaves;
     wave_argmax(held ? sv[lane] : 0.0f, held ? si[lane] : kNoIndex, held && si[lane] != kNoIndex, held && sn[lane] != 0, bv, bi, nan);
     if (tid != 0) return;
     const bool poisoned = nan != 0;
@@ -102,8 +106,11 @@ int launch_argmax_parts(const float* logits, uint64_t stride, uint32_t rows, uin
 
 int launch_argmax_finish(const ArgPart* parts, uint32_t n_parts, uint32_t n_vec, uint32_t* result, int32_t* ids,
                          const uint32_t* ids_slots, int32_t* ids_scatter, uint64_t scatter_len, hipStream_t st) {
-    hipLaunchKernelGGL(k_argmax_finish, dim3(n_vec), dim3(kFinishBlock), 0, st, parts, n_parts, result, ids, ids_slots, ids_scatter,
-                       scatter_len);
+    auto launch = [&](auto kernel, uint32_t block) {
+        hipLaunchKernelGGL(kernel, dim3(n_vec), dim3(block), 0, st, parts, n_parts, result, ids, ids_slots, ids_scatter, scatter_len);
+    };
+    if (n_parts <= kFinishSmallBlock) launch(k_argmax_finish<kFinishSmallBlock>, kFinishSmallBlock);
+    else launch(k_argmax_finish<kFinishBlock>, kFinishBlock);
     return hip_status(hipGetLastError(), "argmax_finish launch");
 }
 

@@ -8,7 +8,7 @@ from test_gpu_parity import host, say, to_dev
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 64, 65, 64 * 64 + 1, 64 * 1024, 64 * 1024 + 3, 64 * 4096 - 1, 64 * 4096 + 70, 700001])
+@pytest.mark.parametrize("n", [1, 64, 65, 64 * 64 + 1, 64 * 256, 64 * 256 + 1, 64 * 1024, 64 * 1024 + 3, 64 * 4096 - 1, 64 * 4096 + 70, 700001])
 def test_argmax_over_parts(hl, dev, n):
     import torch
 
