@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <cstdint>
 #include <cstdlib>
+#include <type_traits>
 
 #include "device.h"
 #include "launch.h"
@@ -25,11 +26,14 @@ using namespace dev;
 // registers. Bound by HBM: the rows' accesses are one line apart per lane, and a thread of a
 // 32-weight format takes several blocks so that it uses most of a line at once. Measured on MI355X,
 // 17408 x 5120, repack / unpack us (bytes moved one by one through a block in scratch memory, and
-// unpack with the blocks of a row side by side, before): Q4_0 61 / 125 -> 37 / 58, Q8_0 121 / 304 ->
-// 52 / 70, Q4_K 23 (its own 16-byte path) / 589 -> 23 / 26, Q5_K 179 / 738 -> 29 / 30, Q6_K 217 / 886
-// -> 39 / 42 (73 MB: 3.7 TB/s read and written), IQ4_XS 139 / 609 -> 25 / 25.
+// unpack with the blocks of a row side by side, before): Q4_0 61 / 125 -> 32 / 58, Q8_0 120 / 304 ->
+// 42 / 70, Q4_K 22 (its own 16-byte path) / 589 -> 18 / 26, Q5_K 174 / 738 -> 21 / 30, Q6_K 223 / 886
+// -> 34 / 42 (73 MB: 4.4 TB/s read and written), IQ4_XS 136 / 609 -> 17 / 25. (With a branch around every load
+// for the rows past the last Q4_K took 22, Q6_K 39 and Q4_K 17408 x 17408 94, against its older path's 86.)
 template <uint32_t T>
 constexpr uint32_t kRepackBlocks = T == kQ4_0 ? 8u : T == kQ8_0 ? 4u : 1u;
+// A matrix that gives too few threads that way to fill the chip takes one block per thread (repack_blocks).
+constexpr uint64_t kRepackThreads = 16384;
 
 __device__ __forceinline__ uint4 ld16(const uint8_t* p) {
     uint4 v;
@@ -63,11 +67,15 @@ __device__ __forceinline__ void nibbles_to_slots(const uint4& a4, const uint4& c
 template <uint32_t T>
 __device__ __forceinline__ void repack_block(const uint8_t* __restrict__ s, bool live, uint8_t* __restrict__ out, const SlabGeom& g,
                                              uint32_t r, uint32_t b) {
-    auto in = [&](uint32_t o) __attribute__((always_inline)) { return live ? ld16(s + o) : uint4{0, 0, 0, 0}; };
+    // (past the last row s is the first row's block: every load is issued without a branch of its own)
+    auto in = [&](uint32_t o) __attribute__((always_inline)) {
+        const uint4 v = ld16(s + o);
+        return uint4{live ? v.x : 0u, live ? v.y : 0u, live ? v.z : 0u, live ? v.w : 0u};
+    };
     auto in2 = [&](uint32_t o) __attribute__((always_inline)) {
-        uint16_t v = 0;
-        if (live) __builtin_memcpy(&v, s + o, 2);
-        return v;
+        uint16_t v;
+        __builtin_memcpy(&v, s + o, 2);
+        return live ? v : (uint16_t)0;
     };
     auto rec = [&](uint64_t off, uint64_t i, uint32_t bytes) __attribute__((always_inline)) { return out + off + (i * 64 + r) * bytes; };
     if constexpr (T == kQ4_0 || T == kQ8_0) {
@@ -82,8 +90,9 @@ __device__ __forceinline__ void repack_block(const uint8_t* __restrict__ s, bool
         }
         *reinterpret_cast<uint16_t*>(rec(g.aux_off, b, 2)) = d;
     } else if constexpr (T == kIQ4_XS) {
-        uint2 hdr{0, 0};
-        if (live) __builtin_memcpy(&hdr, s, 8);
+        uint2 hdr;
+        __builtin_memcpy(&hdr, s, 8);
+        if (!live) hdr = uint2{0, 0};
         uint4 q[8];
 #pragma unroll
         for (uint32_t j = 0; j < 8; ++j) q[j] = in(8 + 16 * j);
@@ -228,10 +237,9 @@ __device__ __forceinline__ void unpack_block(const uint8_t* __restrict__ src, ui
     }
 }
 
-template <uint32_t T>
+template <uint32_t T, uint32_t NB>
 __global__ __launch_bounds__(256) void k_repack_slab(const uint8_t* __restrict__ src, uint64_t src_stride, uint32_t rows, uint32_t cols,
                                                      uint8_t* __restrict__ dst) {
-    constexpr uint32_t NB = kRepackBlocks<T>;
     const SlabGeom g = slab_geom(T, cols);
     const uint32_t nblk = cols / block_elems(T), groups = (nblk + NB - 1) / NB;
     const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -247,10 +255,9 @@ __global__ __launch_bounds__(256) void k_repack_slab(const uint8_t* __restrict__
                             r, b0 + k);
 }
 
-template <uint32_t T>
+template <uint32_t T, uint32_t NB>
 __global__ __launch_bounds__(256) void k_unpack_slab(const uint8_t* __restrict__ src, uint32_t rows, uint32_t cols,
                                                      uint8_t* __restrict__ dst, uint64_t dst_stride) {
-    constexpr uint32_t NB = kRepackBlocks<T>;
     const SlabGeom g = slab_geom(T, cols);
     const uint32_t nblk = cols / block_elems(T), groups = (nblk + NB - 1) / NB;
     const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -425,40 +432,51 @@ int launch_stream_read(const void* p, uint64_t bytes, uint32_t workgroups, uint3
     return hip_status(hipGetLastError(), "stream_read launch");
 }
 
-// Threads of a repack or unpack launch: one per row (of whole slabs) and kRepackBlocks blocks
-template <uint32_t T>
-static dim3 repack_grid(uint32_t rows, uint32_t cols) {
-    const uint64_t groups = (cols / block_elems(T) + kRepackBlocks<T> - 1) / kRepackBlocks<T>;
-    return dim3((uint32_t)((((uint64_t)rows + kSlabRows - 1) / kSlabRows * kSlabRows * groups + 255) / 256));
+// Calls launch(blocks per thread, grid) for a repack or unpack: a thread per row (of whole slabs) and kRepackBlocks
+// blocks, or one block where those are fewer than kRepackThreads (MI355X, Q4_0 with 8 and with 1, us: repack 64 x 17408
+// 4.4 and 2.1, 1000 x 1024 4.1 and 2.2; unpack 64 x 17408 5.8 and 2.4; Q8_0 with 4 and 1: 64 x 17408 4.8 and 2.5).
+template <uint32_t T, typename F>
+static void repack_blocks(uint32_t rows, uint32_t cols, F launch) {
+    const uint64_t padded = ((uint64_t)rows + kSlabRows - 1) / kSlabRows * kSlabRows, nblk = cols / block_elems(T);
+    auto with = [&](auto nb) {
+        const uint64_t threads = padded * ((nblk + nb() - 1) / nb());
+        if (nb() > 1 && threads < kRepackThreads) return false;
+        launch(nb, dim3((uint32_t)((threads + 255) / 256)));
+        return true;
+    };
+    if (!with(std::integral_constant<uint32_t, kRepackBlocks<T>>{})) with(std::integral_constant<uint32_t, 1>{});
+}
+
+// Calls f(integral constant) with the SLAB type
+template <typename F>
+static void with_slab_type(uint32_t type, F f) {
+    switch (type) {
+        case kQ4_0: f(std::integral_constant<uint32_t, kQ4_0>{}); break;
+        case kQ8_0: f(std::integral_constant<uint32_t, kQ8_0>{}); break;
+        case kQ4_K: f(std::integral_constant<uint32_t, kQ4_K>{}); break;
+        case kQ5_K: f(std::integral_constant<uint32_t, kQ5_K>{}); break;
+        case kIQ4_XS: f(std::integral_constant<uint32_t, kIQ4_XS>{}); break;
+        default: f(std::integral_constant<uint32_t, kQ6_K>{}); break;
+    }
 }
 
 int launch_repack_slab(uint32_t type, const uint8_t* src, uint64_t src_stride, uint32_t rows, uint32_t cols,
                        uint8_t* dst, hipStream_t st) {
-#define HALO_MI_RP(T) hipLaunchKernelGGL(k_repack_slab<T>, repack_grid<T>(rows, cols), dim3(256), 0, st, src, src_stride, rows, cols, dst)
-    switch (type) {
-        case kQ4_0: HALO_MI_RP(kQ4_0); break;
-        case kQ8_0: HALO_MI_RP(kQ8_0); break;
-        case kQ4_K: HALO_MI_RP(kQ4_K); break;
-        case kQ5_K: HALO_MI_RP(kQ5_K); break;
-        case kIQ4_XS: HALO_MI_RP(kIQ4_XS); break;
-        default: HALO_MI_RP(kQ6_K); break;
-    }
-#undef HALO_MI_RP
+    with_slab_type(type, [&](auto t) {
+        repack_blocks<t()>(rows, cols, [&](auto nb, dim3 grid) {
+            hipLaunchKernelGGL((k_repack_slab<t(), nb()>), grid, dim3(256), 0, st, src, src_stride, rows, cols, dst);
+        });
+    });
     return hip_status(hipGetLastError(), "repack_slab launch");
 }
 
 int launch_unpack_slab(uint32_t type, const uint8_t* src, uint32_t rows, uint32_t cols, uint8_t* dst,
                        uint64_t dst_stride, hipStream_t st) {
-#define HALO_MI_UP(T) hipLaunchKernelGGL(k_unpack_slab<T>, repack_grid<T>(rows, cols), dim3(256), 0, st, src, rows, cols, dst, dst_stride)
-    switch (type) {
-        case kQ4_0: HALO_MI_UP(kQ4_0); break;
-        case kQ8_0: HALO_MI_UP(kQ8_0); break;
-        case kQ4_K: HALO_MI_UP(kQ4_K); break;
-        case kQ5_K: HALO_MI_UP(kQ5_K); break;
-        case kIQ4_XS: HALO_MI_UP(kIQ4_XS); break;
-        default: HALO_MI_UP(kQ6_K); break;
-    }
-#undef HALO_MI_UP
+    with_slab_type(type, [&](auto t) {
+        repack_blocks<t()>(rows, cols, [&](auto nb, dim3 grid) {
+            hipLaunchKernelGGL((k_unpack_slab<t(), nb()>), grid, dim3(256), 0, st, src, rows, cols, dst, dst_stride);
+        });
+    });
     return hip_status(hipGetLastError(), "unpack_slab launch");
 }
 

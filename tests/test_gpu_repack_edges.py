@@ -4,7 +4,7 @@ rows back without touching what lies between them."""
 import numpy as np
 import pytest
 
-from helpers import BLOCK, NAMES, QUANT_TYPES, dense_rows, make_weights, row_bytes
+from helpers import BLOCK, NAMES, Q4_0, Q8_0, QUANT_TYPES, dense_rows, make_weights, row_bytes
 from test_gpu_parity import host, say, to_dev
 
 pytestmark = pytest.mark.gpu
@@ -36,3 +36,11 @@ def test_repack_and_back(hl, oracle, dev, t, rows, blocks, pad, off):
     assert np.array_equal(back[inside], buf[inside])
     assert np.all(back[~inside] == 0x5A)
 
+
+
+@pytest.mark.parametrize("t", [Q4_0, Q8_0])
+@pytest.mark.parametrize("rows,blocks", [(8193, 9), (16321, 1), (8129, 8)])
+@pytest.mark.parametrize("pad,off", [(0, 0), (5, 3)])
+def test_several_blocks_per_thread(hl, oracle, dev, t, rows, blocks, pad, off):
+    """Enough threads for several blocks each, with a part of them left, and just too few."""
+    test_repack_and_back(hl, oracle, dev, t, rows, blocks, pad, off)
