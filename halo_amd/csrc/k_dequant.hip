@@ -288,13 +288,18 @@ __device__ __forceinline__ bool table_row(const int32_t* ids, uint32_t table_row
     return true;
 }
 
-// Dequantize / GET_ROWS: a block of kDqThreads threads takes kDqElems consecutive elements of one
-// output row (blocks of a row follow each other, so the row's index is one scalar division), four
-// consecutive elements per thread: a wave stores 1 KB at once. Bound by launch and load latency at
-// a prefill chunk's sizes: 512 rows of 5120 from a Q6_K SLAB table 7.9 -> 5.7 us (one thread per
-// 32-element slot stored 4 bytes at a 128-byte pitch), from a GGUF table 8.7 -> 6.5 us (one thread
-// per element with 64-bit divisions); Q4_K 7.2 -> 4.7 and 8.8 -> 6.3.
-constexpr uint32_t kDqThreads = 256, kDqElems = 4 * kDqThreads;
+// Dequantize / GET_ROWS: a block of kDqThreads threads takes E elements of one output row per thread, consecutive
+// ones (blocks of a row follow each other, so the row's index is one scalar division): with four a wave stores
+// 1 KB at once. Bound by launch and load latency at a prefill chunk's sizes: 512 rows of 5120 from a Q6_K SLAB
+// table 7.9 -> 5.7 us (one thread per 32-element slot stored 4 bytes at a 128-byte pitch), from a GGUF table
+// 8.7 -> 6.5 us (one thread per element with 64-bit divisions); Q4_K 7.2 -> 4.7 and 8.8 -> 6.3.
+constexpr uint32_t kDqThreads = 256;
+// Elements of a GGUF call from which a thread takes four: with rows aligned for 16-byte stores, and with others.
+// Below, the chip has threads to spare, and a thread's four byte-wise decodes in a row add latency (MI355X, one and
+// four elements per thread, means of the 16 types, us: 1 x 5120 2.0 and 2.2, 64 x 5120 2.4 and 2.6, 102 x 5120 2.82 and
+// 2.88; on other rows 64 x 5120 2.5 and 3.0, 512 x 2048 4.2 and 4.4; one per thread with 64-bit divisions 2.1, 2.6, 3.05;
+// 2.7, 4.5. From there on four gain: 512 x 2048 aligned 4.0 and 3.5, 4096 x 5120 56 and 30, on other rows 55 and 37).
+constexpr uint64_t kDqQuadElems = 1ull << 20, kDqQuadElemsOther = 1ull << 22;
 
 // Stores w[0..3] at o[i..i+3], of which the first `left` exist; 16-byte stores where the row is aligned.
 __device__ __forceinline__ void store4(float* o, uint32_t i, uint32_t left, const float w[4]) {
@@ -307,22 +312,27 @@ __device__ __forceinline__ void store4(float* o, uint32_t i, uint32_t left, cons
     }
 }
 
-template <uint32_t T>
+template <uint32_t T, uint32_t E>
 __global__ __launch_bounds__(kDqThreads) void k_dequant_gguf(const uint8_t* __restrict__ w, uint64_t w_stride, uint32_t cols,
                                                              uint32_t first_row, uint32_t blocks_per_row,
                                                              float* __restrict__ out, uint64_t out_stride,
                                                              const int32_t* __restrict__ ids, uint32_t table_rows,
                                                              uint32_t* status) {
     const uint32_t r = blockIdx.x / blocks_per_row;
-    const uint32_t i = (blockIdx.x % blocks_per_row) * kDqElems + 4 * threadIdx.x;
+    const uint32_t i = (blockIdx.x % blocks_per_row) * (E * kDqThreads) + E * threadIdx.x;
     if (i >= cols) return;
     uint64_t row;
     if (!table_row(ids, table_rows, first_row, r, i == 0, status, row)) return;
     const uint8_t* p = w + row * w_stride;
-    float v[4];
+    if constexpr (E == 1) {
+        out[r * out_stride + i] = gguf_elem<T>(p, i);
+    } else {
+        static_assert(E == 4);
+        float v[4];
 #pragma unroll
-    for (uint32_t k = 0; k < 4; ++k) v[k] = i + k < cols ? gguf_elem<T>(p, i + k) : 0.0f;
-    store4(out + r * out_stride, i, cols - i, v);
+        for (uint32_t k = 0; k < 4; ++k) v[k] = i + k < cols ? gguf_elem<T>(p, i + k) : 0.0f;
+        store4(out + r * out_stride, i, cols - i, v);
+    }
 }
 
 // Exact fp32 weights 4 k .. 4 k + 3 of slot s of the row at lane r of `slab` (the reference's
@@ -383,7 +393,7 @@ __global__ __launch_bounds__(kDqThreads) void k_dequant_slab(const uint8_t* __re
                                                              uint32_t table_rows, uint32_t* status) {
     const SlabGeom g = slab_geom(T, cols);
     const uint32_t r = blockIdx.x / blocks_per_row;
-    const uint32_t i = (blockIdx.x % blocks_per_row) * kDqElems + 4 * threadIdx.x;
+    const uint32_t i = (blockIdx.x % blocks_per_row) * (4 * kDqThreads) + 4 * threadIdx.x;
     if (i >= cols) return;
     uint64_t row;
     if (!table_row(ids, table_rows, first_row, r, i == 0, status, row)) return;
@@ -496,9 +506,15 @@ static int dequant_blocks(uint32_t n_rows, uint32_t per, uint32_t first_row, flo
 int launch_dequant_gguf(uint32_t type, const uint8_t* w, uint64_t w_stride, uint32_t cols, uint32_t first_row,
                         uint32_t n_rows, float* out, uint64_t out_stride, hipStream_t st, const int32_t* ids,
                         uint32_t table_rows, uint32_t* status) {
-    const uint32_t per = (cols - 1) / kDqElems + 1;
+    const bool aligned = (reinterpret_cast<uintptr_t>(out) % 16 | out_stride % 4) == 0;
+    const bool quads = (uint64_t)n_rows * cols >= (aligned ? kDqQuadElems : kDqQuadElemsOther);
+    const uint32_t per = (cols - 1) / ((quads ? 4 : 1) * kDqThreads) + 1;
     const dim3 block(kDqThreads);
-#define HALO_MI_DQ(T) case T: hipLaunchKernelGGL(k_dequant_gguf<T>, grid, block, 0, st, w, w_stride, cols, first, per, o, out_stride, id, table_rows, status); break
+#define HALO_MI_DQ(T)                                                                                                                                   \
+    case T:                                                                                                                                             \
+        if (quads) hipLaunchKernelGGL((k_dequant_gguf<T, 4>), grid, block, 0, st, w, w_stride, cols, first, per, o, out_stride, id, table_rows, status); \
+        else hipLaunchKernelGGL((k_dequant_gguf<T, 1>), grid, block, 0, st, w, w_stride, cols, first, per, o, out_stride, id, table_rows, status);       \
+        break
     return dequant_blocks(n_rows, per, first_row, out, out_stride, ids, [&](dim3 grid, uint32_t first, float* o, const int32_t* id) {
     switch (type) {
         HALO_MI_DQ(kF32);
@@ -526,7 +542,7 @@ int launch_dequant_gguf(uint32_t type, const uint8_t* w, uint64_t w_stride, uint
 
 int launch_dequant_slab(uint32_t type, const uint8_t* w, uint32_t cols, uint32_t first_row, uint32_t n_rows, float* out,
                         uint64_t out_stride, hipStream_t st, const int32_t* ids, uint32_t table_rows, uint32_t* status) {
-    const uint32_t per = (cols - 1) / kDqElems + 1;
+    const uint32_t per = (cols - 1) / (4 * kDqThreads) + 1;
     const dim3 block(kDqThreads);
 #define HALO_MI_DQ(T) hipLaunchKernelGGL(k_dequant_slab<T>, grid, block, 0, st, w, cols, first, per, o, out_stride, id, table_rows, status)
     return dequant_blocks(n_rows, per, first_row, out, out_stride, ids, [&](dim3 grid, uint32_t first, float* o, const int32_t* id) {

@@ -110,6 +110,29 @@ def test_get_rows_bitwise_and_bad_ids(hl, oracle, dev, t, layout):
     assert isclose_bits(host(out)[:3, :cols], ref[[3, 2, 1]])
 
 
+@pytest.mark.parametrize("t", GGUF_TYPES)
+# one element per thread, four, and four on rows not aligned for 16-byte stores, with part of a block left; and just below
+@pytest.mark.parametrize("n,pad", [(1023, 0), (1024, 0), (1025, 3), (4096, 3)])
+def test_get_rows_many(hl, oracle, dev, t, n, pad):
+    import torch
+
+    rows, cols = 9, (1027 if t in PLAIN_TYPES else 1024)
+    say("get_rows many", NAMES[t], n, pad)
+    buf, stride = make_weights(t, rows, cols, seed=t, stride_pad=4, offset=4)
+    ref = oracle.dequantize_rows(t, buf[4:], rows, cols, stride)
+    wd, ids = to_dev(buf, dev), (np.arange(n) * 5 % rows).astype(np.int32)
+    ids[7], ids[n - 1] = rows, -3
+    ostride = (cols + 3) // 4 * 4 + pad
+    out = torch.full((n, ostride), SENTINEL, dtype=torch.float32, device=dev)
+    status = torch.zeros(1, dtype=torch.int32, device=dev)
+    hl.get_rows(t, hl.Layout.GGUF, wd.data_ptr() + 4, rows, cols, to_dev(ids, dev), n, out, table_stride=stride,
+                out_stride=ostride, status=status)
+    o, good = host(out), (ids >= 0) & (ids < rows)
+    assert isclose_bits(o[good, :cols], ref[ids[good]])
+    assert np.all(o[~good] == SENTINEL) and np.all(o[:, cols:] == SENTINEL)
+    assert int(host(status)[0]) == hl.STATUS_BAD_INDEX
+
+
 def test_get_rows_rejects(hl, dev):
     import torch
 
