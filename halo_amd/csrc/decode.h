@@ -47,22 +47,6 @@ __device__ __forceinline__ void q4k_scales(const uint4& hdr, uint32_t j, float& 
     m1 = h2f(hdr.x >> 16) * (float)m;
 }
 
-// ---- Q6_K slot record -> 6-bit unsigned quants, 4 per dword (byte lanes) --------------------
-// ql: the 16-byte low-nibble record; qh: the 8-byte top-bit record (see q6_qh_byte).
-// Output dword i (0..3) holds elements 4i..4i+3 (lo[i]) and 16+4i..16+4i+3 (hi[i]).
-__device__ __forceinline__ void q6_slot_bytes(const uint4& ql, const uint2& qh, uint32_t lo[4], uint32_t hi[4]) {
-    const uint32_t L[4] = {ql.x, ql.y, ql.z, ql.w};
-    const uint32_t H[2] = {qh.x, qh.y};
-#pragma unroll
-    for (int w = 0; w < 2; ++w) {
-        const uint32_t a = L[2 * w], b = L[2 * w + 1], h = H[w];
-        lo[2 * w] = (a & 0x0F0F0F0Fu) | (h & 0x30303030u);
-        hi[2 * w] = ((a >> 4) & 0x0F0F0F0Fu) | ((h >> 2) & 0x30303030u);
-        lo[2 * w + 1] = (b & 0x0F0F0F0Fu) | ((h << 4) & 0x30303030u);
-        hi[2 * w + 1] = ((b >> 4) & 0x0F0F0F0Fu) | ((h << 2) & 0x30303030u);
-    }
-}
-
 // ---- IQ4_XS ---------------------------------------------------------------------------------
 // The IQ4_NL value table of the GGUF format (ggml's kvalues_iq4nl; the reference's copy is at
 // src/tensor/ggml_tables.h:94-96), four int8 values per dword.

@@ -33,7 +33,9 @@ using namespace dev;
 
 
 
-// Q6_K slot record -> 6-bit quants as bytes, like q6_slot_bytes (decode.h), for the GEMV.
+// Q6_K slot record -> 6-bit unsigned quants, 4 per dword (byte lanes). ql: the 16-byte low-nibble
+// record; qh: the 8-byte top-bit record (see q6_qh_byte). Output dword i (0..3) holds elements
+// 4i..4i+3 (lo[i]) and 16+4i..16+4i+3 (hi[i]).
 __device__ __forceinline__ void q6_slot_bytes_gemv(const uint4& ql, const uint2& qh, uint32_t lo[4], uint32_t hi[4]) {
     const uint32_t L[4] = {ql.x, ql.y, ql.z, ql.w};
     const uint32_t H[2] = {qh.x, qh.y};

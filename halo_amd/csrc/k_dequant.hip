@@ -376,7 +376,7 @@ __device__ __forceinline__ void slab_quad_weights(const uint8_t* __restrict__ sl
         const uint32_t c = iq4_lookup4(nib);
 #pragma unroll
         for (int e = 0; e < 4; ++e) w[e] = dl * (ubyte(c, e) - 128.0f);
-    } else {  // Q6_K: the top bits as q6_slot_bytes places them
+    } else {  // Q6_K: the top bits as q6_slot_bytes_gemv (gemv_device.h) places them
         const uint32_t h = word(g.aux_off + sr * 8 + 4 * (i >> 1));
         const uint32_t top = (high ? ((i & 1u) ? h << 2 : h >> 2) : ((i & 1u) ? h << 4 : h)) & 0x30303030u;
         const int8_t sc = *reinterpret_cast<const int8_t*>(slab + g.sc_off + br * 16 + 2 * (s % 8) + high);
