@@ -215,33 +215,45 @@ __global__ __launch_bounds__(ref_threads<NV>()) void k_gemv_gguf_ref(const uint8
         }
 }
 
-// One vector: the same sums with the products computed ahead by other waves. A lone wave per 8 rows
-// leaves the chip idle (5120 rows: 640 waves on 1024 SIMDs) and pays decode, multiply and add in one
-// dependent stream. Here a workgroup takes 8 rows with one chain wave and kOneProducers producer
-// waves: in round r producer i turns chunk r * kOneProducers + i (kOneChunk elements of K) into
-// products in LDS, one 16-byte quad per lane and slot, and the chain wave adds the round before in
-// order (lane l: sum l % 8 of row l / 8, as above). The chain wave only reads and adds; what bounds
-// the kernel is the producers' instructions (about 28 per slot of 4 x 64 products). Rows' bytes and x
-// are loaded kOneAhead rounds ahead (a round is shorter than a memory round trip). The chain wave's
-// place in the workgroup changes with the workgroup, so every SIMD gets as many of them.
-// Measured on MI355X against k_gemv_gguf_ref with one vector, us: 5120 x 17408 IQ4_NL 66.0 -> 57.6, Q3_K
-// 93.5 -> 76.3, Q6_K 98.1 -> 68.8; 1024 x 5120 20.5 -> 13.9, 29.5 -> 17.5, 30.3 -> 16.6; 6144 x 5120
-// 22.4 -> 19.6, 31.9 -> 25.4, 34.2 -> 23.9; 17408 x 5120 38.4 -> 47.6, 54.4 -> 65.1, 51.7 -> 57.0. So it
-// takes the matrices whose workgroups are all resident at once (3 per CU by their LDS).
+// Few rows and vectors: the same sums with the products computed ahead by other waves, one vector
+// (blockIdx.y) per workgroup. A lone wave per 8 rows leaves the chip idle (5120 rows: 640 waves on 1024
+// SIMDs) and pays decode, multiply and add in one dependent stream. Here a workgroup takes 8 rows with one
+// chain wave and kOneProducers producer waves: in round r producer i turns chunk r * kOneProducers + i
+// (kOneChunk elements of K) into products in LDS, one 16-byte quad per lane and slot, and the chain wave
+// adds the round before in order (lane l: sum l % 8 of row l / 8, as above). Rows' bytes and x are loaded
+// kOneAhead rounds ahead (a round is shorter than a memory round trip). The chain wave's place in the
+// workgroup changes with the workgroup, so every SIMD gets as many of them.
+// What bounds it is the length of a round (1.7 us at 5120 x 17408), not the issue rate: the producers'
+// instructions (about 28 per slot of 4 x 64 products) are 16 of IQ4_NL's 57 us there and the chain's adds 7,
+// but a producer writes a chunk's bytes, waits, reads them, writes the products and meets the barrier
+// one after the other.
+// Measured on MI355X against k_gemv_gguf_ref, us. One vector: 5120 x 17408 IQ4_NL 62 -> 57, Q3_K 92 -> 75, Q6_K
+// 99 -> 70; 1024 x 5120 19 -> 14, 29 -> 17, 30 -> 16; 8192 x 5120 22 -> 22, 33 -> 31, 35 -> 28; 10240 x 5120 27 -> 32,
+// 40 -> 42, 42 -> 39; 17408 x 5120 35 -> 47, 53 -> 62, 52 -> 56. Two vectors of 1024 x 5120: 20 -> 14, 30 -> 18, 30 ->
+// 17; eight of them 28 -> 21, 43 -> 27, 44 -> 24.
 constexpr uint32_t kOneProducers = 2, kOneChunk = 256, kOneAhead = 3;
-constexpr uint32_t kOneMaxRows = 8 * 3 * 256;
+// LDS of a workgroup: 36.9-39.7 KB for the quantized types, 43.5 for the 16-bit ones, 51.7 for F32
+template <uint32_t T>
+constexpr uint32_t one_lds_bytes() {
+    constexpr uint32_t row = (kOneChunk / block_elems(T) * block_bytes(T) + 15) / 16 * 16 + 16;
+    return kOneProducers * (8 * row + 4 * 8 * (kOneChunk / 8 + 4)) + 2 * kOneProducers * (kOneChunk / 32) * 64 * 16;
+}
 
 template <uint32_t T>
 __global__ __launch_bounds__(64 * (kOneProducers + 1)) void k_gemv_gguf_one(const uint8_t* __restrict__ w, uint64_t w_stride,
-                                                                            const float* __restrict__ x, float* __restrict__ y,
-                                                                            uint32_t rows, uint32_t cols) {
+                                                                            const float* __restrict__ x, uint64_t x_stride,
+                                                                            float* __restrict__ y, uint64_t y_stride, uint32_t rows,
+                                                                            uint32_t cols) {
 #pragma clang fp contract(off)
     constexpr uint32_t BE = block_elems(T), BB = block_bytes(T), P = kOneProducers, CH = kOneChunk, CHB = CH / BE * BB;
     constexpr uint32_t PIECES = (CHB + 15) / 16, NLD = (8 * PIECES + 63) / 64;
     constexpr uint32_t RS = PIECES * 16 + 16, XS = CH / 8 + 4, XLD = CH / 64, SLOTS = CH / 32;
+    x += blockIdx.y * x_stride;
+    y += blockIdx.y * y_stride;
     __shared__ __align__(16) uint8_t wl[P][8 * RS];
     __shared__ __align__(16) float xl[P][8 * XS];
     __shared__ float4 prod[2][P][SLOTS][64];
+    static_assert(sizeof(wl) + sizeof(xl) + sizeof(prod) == one_lds_bytes<T>());
     const uint32_t lane = threadIdx.x & 63u, j = lane & 7u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t role = (wave + P + 1 - blockIdx.x % (P + 1)) % (P + 1);  // P: the chain wave; else producer
@@ -391,40 +403,44 @@ void launch_ref_nv(const RefArgs& a, uint32_t t0, uint32_t n, hipStream_t st) {
 
 template <uint32_t T>
 void launch_ref(const RefArgs& a, uint32_t n_vec, hipStream_t st) {
-    // Large groups decode least and small ones fill the chip soonest: a group's time hardly depends on
-    // its rows until there is about a wave per SIMD (1024). So: groups of 16 vectors with two rows per lane
-    // where those are 1024 waves; one of 8 for what is left of a large matrix; then groups of 4, or of 2
-    // while 4 would be fewer than 1024 waves. Measured on MI355X against groups of 16 and 8 everywhere, us:
-    // IQ4_NL 5120 x 17408 at 4 / 8 / 16 / 32 vectors 177 / 242 / 464 / 461 -> 110 / 184 / 211 / 383; Q3_K 1024 x
-    // 5120 45 / 55 / 130 / 131 -> 40 / 41 / 41 / 48; F16 6144 x 5120 40 / 78 / 137 / 143 -> 31 / 42 / 82 / 124.
-    uint32_t t = 0;  // vectors done
-    const uint32_t g16 = n_vec / 16 + (n_vec % 16 > 8 ? 1 : 0);
-    if ((uint64_t)a.rows * g16 >= 16 * 1024) {
-        t = std::min(n_vec, 16 * g16);
-        launch_ref_nv<T, 16, 2>(a, 0, t, st);
-    }
-    if (n_vec - t > 4 && n_vec - t <= 8 && a.rows >= 32 * 1024) {
-        launch_ref_nv<T, 8, 2>(a, t, n_vec - t, st);
-        t = n_vec;
-    }
-    if (n_vec - t > 2) {
-        const uint32_t left = n_vec - t;
-        if ((uint64_t)a.rows * ((left + 1) / 4) >= 8 * 1024) {
-            const uint32_t n = std::min(left, (left + 1) / 4 * 4);  // the last group may be of 3
-            launch_ref_nv<T, 4, 1>(a, t, n, st);
-            t += n;
+    // Large vector groups decode least and small ones fill the chip soonest: a group's time hardly depends
+    // on its rows until there is about a wave per SIMD (1024). What decides is therefore the call's work in
+    // units of 8 rows of one vector. While its products-ahead workgroups are all resident at once (four per CU by
+    // the LDS of the quantized types, three for the others; 256 CUs) they win, then groups of 1, 2 and 4 vectors
+    // in turn, but for the types that decode slowest: those skip the groups of one and go to 4 sooner.
+    // Groups of 16 with two rows per lane take over at 1024 waves of them, one of 8 what is left of a large matrix.
+    // Groups of one and two take every vector (a launch of its own costs the whole chain again); beside groups of
+    // 4, one or two vectors left over go on their own (three fill a group).
+    // Measured on MI355X, us, Q4_K of 5120 columns either side of each line: 1024 units ahead 19, groups of one 23;
+    // 1280 31 and 25; 2048 groups of one 27, of two 33; 3072 47 and 37 (2560: Q4_K 34 and 36, but Q5_0 51 and 47); 6144 of
+    // two 48, of four 47; 7680 70 and 48. Slow types: 1280 units of Q3_K 5120 x 1024 ahead / of one / of two 13.1 / 13.9 /
+    // 12.8; 4096 units of two and four IQ3_S 81 and 60, Q6_K 54 and 47, but Q5_K 44 and 58, Q8_0 39 and 65. Against
+    // the products ahead for one vector only, groups of two next and groups of four from 4096 units on: 0.77x the
+    // time over 16 types, 16 sizes and 1 to 64 vectors (IQ3_S 1024 x 5120 at two 67 -> 22), none slower by more than 4-6%.
+    constexpr bool kSlow = T == kQ3_K || T == kQ6_K || T == kIQ3_S;
+    constexpr uint64_t kAhead = 256 * (163840 / one_lds_bytes<T>()), kOnes = kSlow ? 0 : 2048, kTwos = 6144;
+    const uint64_t w = (a.rows - 1) / 8 + 1;  // units of one vector
+    for (uint32_t t = 0; t < n_vec;) {
+        const uint32_t left = n_vec - t, g16 = left / 16 + (left % 16 > 8 ? 1 : 0), g4 = (left + 1) / 4;
+        const bool fours = left > 2 && (kSlow ? (uint64_t)a.rows * g4 >= 8 * 1024 : w * (left + left % 2) > kTwos);
+        uint32_t n = left;
+        if ((uint64_t)a.rows * g16 >= 16 * 1024) {
+            n = std::min(left, 16 * g16);
+            launch_ref_nv<T, 16, 2>(a, t, n, st);
+        } else if (left > 4 && left <= 8 && a.rows >= 32 * 1024) {
+            launch_ref_nv<T, 8, 2>(a, t, n, st);
+        } else if (w * left <= kAhead) {
+            hipLaunchKernelGGL((k_gemv_gguf_one<T>), dim3((uint32_t)w, n), dim3(64 * (kOneProducers + 1)), 0, st, a.w, a.w_stride,
+                               a.x + (uint64_t)t * a.x_stride, a.x_stride, a.y + (uint64_t)t * a.y_stride, a.y_stride, a.rows, a.cols);
+        } else if (w * left <= kOnes || left == 1) {
+            launch_ref_nv<T, 1, 1>(a, t, n, st);
+        } else if (!fours) {
+            launch_ref_nv<T, 2, 1>(a, t, n, st);
         } else {
-            launch_ref_nv<T, 2, 1>(a, t, left / 2 * 2, st);
-            t += left / 2 * 2;
+            n = std::min(left, 4 * g4);
+            launch_ref_nv<T, 4, 1>(a, t, n, st);
         }
-    }
-    if (n_vec - t == 2) {
-        launch_ref_nv<T, 2, 1>(a, t, 2, st);
-    } else if (n_vec - t == 1) {
-        if (a.rows <= kOneMaxRows)
-            hipLaunchKernelGGL((k_gemv_gguf_one<T>), dim3((a.rows - 1) / 8 + 1), dim3(64 * (kOneProducers + 1)), 0, st, a.w, a.w_stride,
-                               a.x + (uint64_t)t * a.x_stride, a.y + (uint64_t)t * a.y_stride, a.rows, a.cols);
-        else launch_ref_nv<T, 1, 1>(a, t, 1, st);
+        t += n;
     }
 }
 

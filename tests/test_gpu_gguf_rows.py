@@ -69,8 +69,8 @@ def test_infinities_and_nan(hl, oracle, dev, t):
 @pytest.mark.parametrize("t", GGUF_TYPES)
 @pytest.mark.parametrize("rows,cols", [(1, 256), (8, 512), (17, 768), (9, 4608), (6144, 256), (6145, 256)])
 def test_one_vector_rounds(hl, oracle, dev, t, rows, cols):
-    """One vector with the products made ahead (up to 6144 rows): fewer chunks than producers, an odd last
-    round, more rounds than are loaded ahead, and the rows on either side of the rule."""
+    """One vector with the products made ahead (6144 rows and more): fewer chunks than producers, an odd last
+    round, more rounds than are loaded ahead, and the 16- and 32-bit types' rows on either side of the rule."""
     check(hl, oracle, dev, t, rows, cols, 1)
 
 
@@ -79,3 +79,14 @@ def test_one_vector_rounds(hl, oracle, dev, t, rows, cols):
 def test_groups_of_four(hl, oracle, dev, t, n_vec):
     """Enough rows for groups of four vectors (a last one of three, and what two and one are left)."""
     check(hl, oracle, dev, t, 8200, 256, n_vec)
+
+
+# (rows, vectors) at and just past each line of the choice of a group
+LINES = [(8192, 1), (8193, 1), (1024, 8), (1025, 8), (768, 8), (769, 8), (8192, 2), (8193, 2), (24577, 1), (24577, 2),
+         (8192, 3), (8191, 3), (12288, 4), (12289, 4), (12281, 3), (16385, 3), (12289, 6), (1, 1024), (1, 1025), (8, 6145)]
+
+
+@pytest.mark.parametrize("t", [Q3_K, IQ4_NL, F16])
+@pytest.mark.parametrize("rows,n_vec", LINES)
+def test_either_side_of_the_lines(hl, oracle, dev, t, rows, n_vec):
+    check(hl, oracle, dev, t, rows, 256, n_vec)
