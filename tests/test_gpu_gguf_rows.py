@@ -81,6 +81,22 @@ def test_groups_of_four(hl, oracle, dev, t, n_vec):
     check(hl, oracle, dev, t, 8200, 256, n_vec)
 
 
+# (rows, vectors): groups of 1 or 2, of 2, of 4 and what is left, of 16 and what is left, of 8
+EVERY_GROUP = [(233, 37), (577, 37), (1361, 38), (8193, 37), (32769, 7)]
+
+
+@pytest.mark.parametrize("t", GGUF_TYPES)
+@pytest.mark.parametrize("rows,n_vec", EVERY_GROUP)
+def test_chunks_of_every_group(hl, oracle, dev, t, rows, n_vec):
+    """Every vector group over several chunks of K and a part of one: the two x buffers are used again, by the
+    four waves that share them for 8 and 16 vectors, at an odd alignment and strides."""
+    if rows > 2000 and t not in (Q3_K, Q6_K, IQ4_NL, Q8_0, F16, F32):
+        pytest.skip("the large shapes run for six types")
+    be = BLOCK[t][0]
+    pad, off = (4, 4) if t == F32 else (3, 1)
+    check(hl, oracle, dev, t, rows, 1280 if be == 256 else 1312 if be == 32 else 1291, n_vec, pad=pad, off=off, xp=1, yp=5)
+
+
 # (rows, vectors) at and just past each line of the choice of a group
 LINES = [(8192, 1), (8193, 1), (1024, 8), (1025, 8), (768, 8), (769, 8), (8192, 2), (8193, 2), (24577, 1), (24577, 2),
          (8192, 3), (8191, 3), (12288, 4), (12289, 4), (12281, 3), (16385, 3), (12289, 6), (1, 1024), (1, 1025), (8, 6145)]
