@@ -101,6 +101,11 @@ bool is_pinned(const void* p) {
     return attr.type == hipMemoryTypeHost;
 }
 
+// Whether the copy engine reads the part's rows where they are: dense, in pinned memory.
+bool read_directly(const halo_mi_upload_part& part, uint64_t rb) {
+    return (part.src_stride == 0 || part.src_stride == rb) && is_pinned(part.src);
+}
+
 // One contiguous byte range to copy into the pinned buffer.
 struct Piece {
     const uint8_t* src;
@@ -170,7 +175,6 @@ int halo_mi_upload_tensors(const halo_mi_upload_tensor* tensors, uint32_t n, uin
     const char* op = "upload_tensors";
     if (n == 0) return HALO_MI_OK;
     if (!tensors) return set_error(HALO_MI_E_KERNEL, "%s: null tensor list", op);
-    const bool pick_chunk = chunk_bytes == 0;
     if (host_threads == 0) host_threads = std::max(1u, std::min(8u, std::thread::hardware_concurrency()));
     // validation
     uint64_t total_bytes = 0;
@@ -196,10 +200,21 @@ int halo_mi_upload_tensors(const halo_mi_upload_tensor* tensors, uint32_t n, uin
     }
     // The first chunk's gather and the last one's repack overlap nothing, so a load of few chunks
     // wants small ones; but a gather starts a thread per 4 MiB of its chunk, and a long load is
-    // fastest with the most (MI355X, pageable memory: a layer's 195 MB FFN in 64 / 28 / 24 / 20 / 16 /
-    // 12 MiB chunks 4.39 / 4.24 / 4.13 / 4.13 / 4.29 / 5.40 ms; 9.4 GB in 64 / 32 / 24 MiB chunks 55.4 /
-    // 54.7 / 54.5 GB/s).
-    if (pick_chunk) chunk_bytes = total_bytes <= (1ull << 30) ? 24ull << 20 : 64ull << 20;
+    // fastest with the most (MI355X, pageable memory, ms in 64 and 24 MiB chunks: 60 MiB 1.71 and 1.55, 200
+    // 4.52 and 4.31, 400 8.25 and 8.22, 700 14.02 and 14.06, 1000 19.74 and 19.79, 2000 38.5 and 39.0, 4000 76.2 and
+    // 77.3; 195 MB in 20 / 16 / 12 MiB chunks 4.13 / 4.29 / 5.40). A load that gathers nothing wants the large ones at
+    // every size (pinned: 60 MiB 1.17 and 1.19, 200 3.81 and 3.89, 1000 18.9 and 19.3).
+    if (chunk_bytes == 0) {
+        const auto gathers = [&] {
+            for (uint32_t i = 0; i < n; ++i)
+                for (uint32_t p = 0; p < tensors[i].n_parts; ++p)
+                    if (const halo_mi_upload_part& part = tensors[i].parts[p];
+                        part.rows && tensors[i].cols && !read_directly(part, halo_mi_row_bytes(tensors[i].type, tensors[i].cols)))
+                        return true;
+            return false;
+        };
+        chunk_bytes = total_bytes <= (512ull << 20) && gathers() ? 24ull << 20 : 64ull << 20;
+    }
     uint64_t slot_bytes = 0;  // the largest chunk (whole slabs of one tensor)
     for (uint32_t i = 0; i < n; ++i) {
         const uint64_t rb = halo_mi_row_bytes(tensors[i].type, tensors[i].cols);
@@ -256,8 +271,7 @@ int halo_mi_upload_tensors(const halo_mi_upload_tensor* tensors, uint32_t n, uin
         // a dense part in pinned memory is read by the copy engine directly
         std::vector<uint8_t> direct(t.n_parts);
         for (uint32_t p = 0; p < t.n_parts; ++p)
-            direct[p] = t.parts[p].rows && (t.parts[p].src_stride == 0 || t.parts[p].src_stride == rb) &&
-                        is_pinned(t.parts[p].src);
+            direct[p] = t.parts[p].rows && read_directly(t.parts[p], rb);
         for (uint64_t r0 = 0; r0 < rows; r0 += chunk_rows, ++chunk) {
             const uint32_t s = (uint32_t)(chunk % nslots);
             const uint64_t nr = std::min<uint64_t>(chunk_rows, rows - r0);

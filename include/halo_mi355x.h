@@ -465,8 +465,8 @@ int halo_mi_unpack_slab_host(uint32_t type, const void* src, uint32_t rows, uint
  *   parts[i].src: host rows, src_stride bytes apart (0 = row_bytes); any host memory.
  *   dst: device memory of halo_mi_slab_bytes(type, sum of the parts' rows, cols) bytes,
  *        16-byte aligned; destinations must not overlap.
- *   chunk_bytes: rows move in chunks of about this size (0 = 24 MiB for a load of up to 1 GiB, else
- *     64 MiB), whole slabs of one tensor;
+ *   chunk_bytes: rows move in chunks of about this size (0 = 24 MiB for a load of up to 512 MiB
+ *     that is not all dense pinned memory, else 64 MiB), whole slabs of one tensor;
  *   host_threads: threads that gather a chunk into pinned memory (0 = up to 8).
  * A three-stage pipeline over 4 chunk slots: the host gathers chunk i + 2 into pinned memory
  * while the copy engine moves chunk i + 1 (on a stream of its own) and `stream` repacks chunk i.

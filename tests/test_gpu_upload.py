@@ -59,7 +59,7 @@ def test_upload_tensors_fused_parts_bitwise(hl, dev, chunk_slabs, threads):
 
 
 def test_upload_tensors_large_default_chunks(hl, dev):
-    """17408 x 5120 Q4_K (50 MB) in 64 MiB chunks, compared with the device repack."""
+    """17408 x 5120 Q4_K (50 MB) in chunks of the default size, compared with the device repack."""
     import torch
 
     t, rows, cols = Q4_K, 17408, 5120
@@ -69,6 +69,28 @@ def test_upload_tensors_large_default_chunks(hl, dev):
     hl.upload_tensors([(t, cols, [(w, rows)], dst)])
     ref = torch.zeros_like(dst)
     hl.repack_slab(t, to_dev(w, dev), rows, cols, ref)
+    assert torch.equal(dst, ref)
+
+
+@pytest.mark.parametrize("case", ["pinned", "pinned rows apart", "pinned and pageable"])
+def test_upload_tensors_default_chunks_of_pinned_rows(hl, dev, case):
+    """The default chunk follows whether any part has to be gathered: 35 MB of rows that are all dense in pinned
+    memory, rows apart in it, and one part of each."""
+    import torch
+
+    t, rows, cols = Q6_K, 8200, 5120
+    say("upload_tensors pinned", case)
+    rb = row_bytes(t, cols)
+    gap = 16 if case == "pinned rows apart" else 0
+    w = torch.empty((rows, rb + gap), dtype=torch.uint8, pin_memory=True).numpy()
+    w[:] = np.random.default_rng(9).integers(0, 256, size=w.shape, dtype=np.uint8)
+    dense = np.ascontiguousarray(w[:, :rb])
+    cut = 3001 if case == "pinned and pageable" else rows
+    parts = [(w, cut, rb + gap)] + ([(dense[cut:], rows - cut)] if cut < rows else [])
+    dst = torch.zeros(hl.slab_bytes(t, rows, cols), dtype=torch.uint8, device=dev)
+    hl.upload_tensors([(t, cols, parts, dst)])
+    ref = torch.zeros_like(dst)
+    hl.repack_slab(t, to_dev(dense, dev), rows, cols, ref)
     assert torch.equal(dst, ref)
 
 
