@@ -105,12 +105,12 @@ __global__ __launch_bounds__(BLOCK) void k_rms_norm_rows(const float* x, uint64_
     }
 }
 
-template <uint32_t PT>
-__global__ __launch_bounds__(kNormBlock) void k_rms_inv_rows(const float* __restrict__ x, uint64_t x_stride,
+template <uint32_t BLOCK, uint32_t PT>
+__global__ __launch_bounds__(BLOCK) void k_rms_inv_rows(const float* __restrict__ x, uint64_t x_stride,
                                                              uint32_t cols, float eps, float* __restrict__ inv) {
     __shared__ float lds[kNormLds];
     float v[PT];
-    const float s = row_rms_inv<kNormBlock, PT>(x + (uint64_t)blockIdx.x * x_stride, cols, eps, lds, v, []() {});
+    const float s = row_rms_inv<BLOCK, PT>(x + (uint64_t)blockIdx.x * x_stride, cols, eps, lds, v, []() {});
     if (threadIdx.x == 0) inv[blockIdx.x] = s;
 }
 
@@ -246,9 +246,16 @@ int launch_norm_to_frag(const float* x, uint64_t x_stride, uint32_t n_vec, uint3
 int launch_rms_inv(const float* x, uint64_t x_stride, uint32_t rows, uint32_t cols, float eps, float* inv,
                    hipStream_t st) {
     if (rows == 0 || cols == 0) return HALO_MI_OK;
-    with_loads(cols, [&](auto pt) {
-        hipLaunchKernelGGL(k_rms_inv_rows<pt()>, dim3(rows), dim3(kNormBlock), 0, st, x, x_stride, cols, eps, inv);
-    });
+    auto launch = [&](auto kernel, uint32_t block) {
+        hipLaunchKernelGGL(kernel, dim3(rows), dim3(block), 0, st, x, x_stride, cols, eps, inv);
+    };
+    // A CU holds three workgroups of 512 threads, or four of 256, which take longer for a row: those where they
+    // save a round (MI355X, what the whole 64-row GEMM of normed x takes with 512 and 256 threads, us: 10240 columns
+    // 768 rows 37.2 and 38.0, 800 43.0 and 39.2, 1024 45.9 and 41.3, 1100 48.1 and 48.0; 12288 columns 1500 rows 85.3
+    // and 85.9, 1024 49.7 and 44.6).
+    const bool many = cols > 6144 && (rows + 767) / 768 > (rows + 1023) / 1024;
+    if (many) launch(k_rms_inv_rows<kNormManyBlock, 32>, kNormManyBlock);
+    else with_loads(cols, [&](auto pt) { launch(k_rms_inv_rows<kNormBlock, pt()>, kNormBlock); });
     return hip_status(hipGetLastError(), "rms_inv launch");
 }
 

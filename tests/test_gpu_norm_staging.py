@@ -1,5 +1,5 @@
 """The GEMM's x staging with the fused norm: bitwise RMS_NORM and then the same GEMM, over the widths its one
-launch takes (and one past them), row counts that leave part of a workgroup's rows or of an M tile as padding,
+launch takes (and past them, on either side of the rows where that form's workgroups get smaller), row counts that leave part of a workgroup's rows or of an M tile as padding,
 strided rows, and rows of zeros, infinities and NaN."""
 import numpy as np
 import pytest
@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("cols,n_vec", [(32, 10), (256, 9), (2048, 33), (2080, 13), (5120, 65), (5120, 200), (6144, 31),
-                                        (8192, 130), (8224, 12)])
+                                        (8192, 130), (8224, 12), (8448, 768), (8448, 769), (8224, 1024), (8448, 1025)])
 @pytest.mark.parametrize("variant", [0, 3])
 def test_staged_norm_is_rms_norm_then_gemm(hl, dev, cols, n_vec, variant):
     import torch
