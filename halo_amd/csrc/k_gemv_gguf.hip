@@ -407,7 +407,8 @@ void launch_ref(const RefArgs& a, uint32_t n_vec, hipStream_t st) {
     // on its rows until there is about a wave per SIMD (1024). What decides is therefore the call's work in
     // units of 8 rows of one vector. While its products-ahead workgroups are all resident at once (four per CU by
     // the LDS of the quantized types, three for the others; 256 CUs) they win, then groups of 1, 2 and 4 vectors
-    // in turn, but for the types that decode slowest: those skip the groups of one and go to 4 sooner.
+    // in turn. The types that decode slowest skip the groups of one; the 256-element blocks but Q5_K's, whose
+    // decoding outweighs what a group of four adds, go to 4 sooner.
     // Groups of 16 with two rows per lane take over at 1024 waves of them, one of 8 what is left of a large matrix.
     // Groups of one and two take every vector (a launch of its own costs the whole chain again); beside groups of
     // 4, one or two vectors left over go on their own (three fill a group).
@@ -416,13 +417,13 @@ void launch_ref(const RefArgs& a, uint32_t n_vec, hipStream_t st) {
     // two 48, of four 47; 7680 70 and 48. Slow types: 1280 units of Q3_K 5120 x 1024 ahead / of one / of two 13.1 / 13.9 /
     // 12.8; 4096 units of two and four IQ3_S 81 and 60, Q6_K 54 and 47, but Q5_K 44 and 58, Q8_0 39 and 65. Against
     // the products ahead for one vector only, groups of two next and groups of four from 4096 units on: 0.77x the
-    // time over 16 types, 16 sizes and 1 to 64 vectors (IQ3_S 1024 x 5120 at two 67 -> 22), none slower by more than 4-6%.
-    constexpr bool kSlow = T == kQ3_K || T == kQ6_K || T == kIQ3_S;
+    // time over 16 types, 16 sizes and 1 to 64 vectors (IQ3_S 1024 x 5120 at two 67 -> 22), none slower by more than 4%.
+    constexpr bool kSlow = T == kQ3_K || T == kQ6_K || T == kIQ3_S, kSooner = block_elems(T) == 256 && T != kQ5_K;
     constexpr uint64_t kAhead = 256 * (163840 / one_lds_bytes<T>()), kOnes = kSlow ? 0 : 2048, kTwos = 6144;
     const uint64_t w = (a.rows - 1) / 8 + 1;  // units of one vector
     for (uint32_t t = 0; t < n_vec;) {
         const uint32_t left = n_vec - t, g16 = left / 16 + (left % 16 > 8 ? 1 : 0), g4 = (left + 1) / 4;
-        const bool fours = left > 2 && (kSlow ? (uint64_t)a.rows * g4 >= 8 * 1024 : w * (left + left % 2) > kTwos);
+        const bool fours = left > 2 && (kSooner ? (uint64_t)a.rows * g4 >= 8 * 1024 : w * (left + left % 2) > kTwos);
         uint32_t n = left;
         if ((uint64_t)a.rows * g16 >= 16 * 1024) {
             n = std::min(left, 16 * g16);
